@@ -210,6 +210,36 @@ def test_gate_matvec(torch_gpu):
     np.testing.assert_allclose(y.cpu().numpy(), ref, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("T,E,hidden,shared,off", [
+    (1, 60, 2048, True, 0), (4, 7, 136, False, 0), (5, 60, 2056, True, 0), (16, 128, 4096, True, 0),
+    (17, 60, 2048, True, 0), (17, 16, 8, True, 0), (33, 15, 2056, False, 0), (130, 128, 4104, True, 0),
+    (20, 60, 100, True, 0), (20, 60, 2048, True, 1), (3, 5, 1, True, 0),
+])
+def test_gate_matvec_sizes(torch_gpu, T, E, hidden, shared, off):
+    """Both gate kernels at the edges of their tiles (16 tokens, 16 rows, 128
+    k) and the unaligned form, against the float64 product.  Bound: at most
+    hidden / 128 + 24 fp32 roundings lie on any term's way into its sum."""
+    from fastllm_py import _native as nat
+
+    torch = torch_gpu
+    g = torch.Generator(device="cuda").manual_seed(T * 1000 + E)
+    buf = torch.randn(T * hidden + off, generator=g, device="cuda")
+    x = buf[off:].view(T, hidden)
+    gw = (torch.randn(E, hidden, generator=g, device="cuda") * 0.1).half()
+    sw = (torch.randn(hidden, generator=g, device="cuda") * 0.1).half()
+    logits = torch.full((T * E + 8,), float("nan"), device="cuda")
+    slog = torch.full((T + 8,), float("nan"), device="cuda")
+    rc = nat.lib().fastllm_gate_matvec(nat.ptr(x), nat.ptr(gw), nat.ptr(sw) if shared else None, nat.ptr(logits),
+                                       nat.ptr(slog) if shared else None, T, E, hidden, nat.current_stream_handle())
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert torch.isnan(logits[T * E:]).all() and torch.isnan(slog[T if shared else 0:]).all()
+    for got, w in [(logits[:T * E].view(T, E), gw)] + ([(slog[:T, None], sw[None])] if shared else []):
+        err = (got.double() - x.double() @ w.double().T).abs()
+        bound = (hidden / 128 + 24) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        assert (err <= bound).all()
+
+
 # ------------------------------------------------------------------ router
 @pytest.mark.parametrize("name", ["qwen15moe_t1", "qwen15moe_t16", "qwen3moe_t512", "deepseek_t32",
                                   "ties_e60_k4", "ties_e128_k8", "ties_e256_k16", "ties_groups"])
