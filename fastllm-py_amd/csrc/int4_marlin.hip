@@ -26,6 +26,7 @@
 #include "device.cuh"
 #include "gemv_common.cuh"
 #include "int4_common.cuh"
+#include "int4_gemm.cuh"
 
 namespace {
 
@@ -940,7 +941,9 @@ __global__ __launch_bounds__(64 * kCsWaves) void int4_gemv_cs(const f16* __restr
     }
 }
 
-// Prefill-shaped GEMM (M > 64, K % 128 == 0) on the matrix cores.
+// Prefill-shaped GEMM of group-32 weights (M > 64, K % 128 == 0) on the
+// matrix cores; group 128 takes int4_gemm_g128 (int4_gemm.hip).  The figures
+// below were taken with group-128 weights, which this kernel served then.
 //
 // Workgroup tile 64 (m) x 256 (n): eight waves side by side along n, each
 // with a 64 x 32 wave tile (4 m-tiles x 2 n-tiles of 16 x 16 fp32
@@ -1000,12 +1003,11 @@ FL_DEV f16x8 dequant_word_scaled(uint32_t w, uint32_t zlo, uint32_t zhi, f16x2 s
     return bitcast<f16x8>(r);
 }
 
-template <bool G32>
 __global__ __launch_bounds__(512) void int4_gemm_mfma(
     const f16* __restrict__ A, const uint32_t* __restrict__ Wq, const uint16_t* __restrict__ S,
     const uint32_t* __restrict__ Z, f16* __restrict__ C, int M, int N, int K) {
     constexpr int D = kGemmAhead, NS = kGemmStages;
-    constexpr int SPB = G32 ? 4 : 1;  // group rows per block
+    constexpr int SPB = 4;  // group rows per block
     // DMA loads per block and wave: 2 A fragments, 2 B tiles, 2 scale/zero
     // pieces (3 * SPB pieces are needed; waves past them repeat one)
     constexpr int LPB = 2 + 2 + 2;
@@ -1016,7 +1018,7 @@ __global__ __launch_bounds__(512) void int4_gemm_mfma(
     const int nkb = K >> 7;
     const int zwords = N >> 3;
     const int ntiles = N >> 4;
-    const int G = K / (G32 ? 32 : 128);
+    const int G = K / 32;
 
     const int nblk = (N + kGemmBN - 1) / kGemmBN, mblk = (M + kGemmBM - 1) / kGemmBM;
     const int total = nblk * mblk;
@@ -1152,9 +1154,8 @@ __global__ __launch_bounds__(512) void int4_gemm_mfma(
                 }
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    const int g = G32 ? j : 0;
-                    const f16x8 b = dequant_word_scaled(wv[t][j], zl[t][g], zh[t][g],
-                                                        f16x2{sc[t][g], sc[t][g]});
+                    const f16x8 b = dequant_word_scaled(wv[t][j], zl[t][j], zh[t][j],
+                                                        f16x2{sc[t][j], sc[t][j]});
 #pragma unroll
                     for (int mt = 0; mt < 4; ++mt) acc[mt][t] = mfma_f16(a[j & 1][mt], b, acc[mt][t]);
                 }
@@ -1179,14 +1180,9 @@ __global__ __launch_bounds__(512) void int4_gemm_mfma(
 }
 
 hipError_t launch_gemm_mfma(const f16* A, const uint32_t* Wq, const uint16_t* S, const uint32_t* Z,
-                            f16* C, int M, int N, int K, bool g32, hipStream_t stream) {
+                            f16* C, int M, int N, int K, hipStream_t stream) {
     const int tiles = ((N + kGemmBN - 1) / kGemmBN) * ((M + kGemmBM - 1) / kGemmBM);
-    if (g32)
-        hipLaunchKernelGGL((int4_gemm_mfma<true>), dim3(tiles), dim3(512), kGemmLds, stream, A, Wq,
-                           S, Z, C, M, N, K);
-    else
-        hipLaunchKernelGGL((int4_gemm_mfma<false>), dim3(tiles), dim3(512), kGemmLds, stream, A, Wq,
-                           S, Z, C, M, N, K);
+    hipLaunchKernelGGL(int4_gemm_mfma, dim3(tiles), dim3(512), kGemmLds, stream, A, Wq, S, Z, C, M, N, K);
     return hipGetLastError();
 }
 
@@ -1463,7 +1459,18 @@ bool int4_marlin_abi_gemm(const void* a, const uint32_t* q, const void* scales,
     const bool g32 = group_size == 32;
     const f16* A = static_cast<const f16*>(a);
     f16* Cp = static_cast<f16*>(c);
-    if (M > kGemmMfmaMinM && K % 128 == 0 && (size_t)N * K / 2 < (1ull << 31)) {
+    const int rows = M > 16 && !g32 && (size_t)N * K / 2 < (1ull << 31) ? int4_gemm_rows(K) : 0;
+    if (rows > 0) {
+        for (int m0 = 0; m0 < M; m0 += rows) {
+            const int Mc = (M - m0) < rows ? (M - m0) : rows;
+            if (!report(int4_gemm_g128(A + (size_t)m0 * K, q, static_cast<const uint16_t*>(scales), zeros,
+                                       Cp + (size_t)m0 * N, Mc, N, K, stream),
+                        "FastllmCudaMarlinHalfInt4Gemm"))
+                return false;
+        }
+        return true;
+    }
+    if (M > kGemmMfmaMinM && g32 && K % 128 == 0 && (size_t)N * K / 2 < (1ull << 31)) {
         // the kernel addresses A through a 32-bit buffer range: launch rows in
         // chunks (multiples of its 64-row tile) of fewer than 2^31 bytes
         const size_t rows_cap = ((1ull << 31) - 1) / ((size_t)K * 2);
@@ -1471,7 +1478,7 @@ bool int4_marlin_abi_gemm(const void* a, const uint32_t* q, const void* scales,
         for (int m0 = 0; m0 < M; m0 += mchunk) {
             const int Mc = (M - m0) < mchunk ? (M - m0) : mchunk;
             if (!report(launch_gemm_mfma(A + (size_t)m0 * K, q, static_cast<const uint16_t*>(scales),
-                                         zeros, Cp + (size_t)m0 * N, Mc, N, K, g32, stream),
+                                         zeros, Cp + (size_t)m0 * N, Mc, N, K, stream),
                         "FastllmCudaMarlinHalfInt4Gemm"))
                 return false;
         }

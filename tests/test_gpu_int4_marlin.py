@@ -197,6 +197,43 @@ def test_gemm_mfma_parity(torch_gpu, M, K, N, gs):
     assert err < TOL, err
 
 
+# every tile shape of the kernel above 16 rows, at ragged rows, ragged columns
+# (N % 96, % 128, % 192 and % 256 != 0) and fewer k blocks than k groups
+@pytest.mark.parametrize("M,K,N", [
+    (17, 128, 64), (40, 1152, 320), (64, 1024, 4096),   # 32 x 32, eight k groups
+    (40, 256, 8128), (33, 640, 8128),                   # 32 x 64
+    (17, 128, 24512), (31, 896, 24512),                 # 32 x 96
+    (64, 128, 24512), (41, 640, 24512),                 # 64 x 96
+    (900, 384, 24512),                                  # 128 x 256
+    (512, 128, 24512), (511, 384, 24512),               # 256 x 192
+    (192, 256, 24512),                                  # 128 x 128
+    (100, 128, 24512), (65, 384, 24512),                # 128 x 128, two k groups
+    (65, 128, 64), (129, 1152, 192), (250, 640, 6080),  # 64 x 128, four k groups
+])
+def test_gemm_tile_shapes(torch_gpu, M, K, N):
+    """Against the float64 product of the same payload.  Bound: the result's
+    rounding to fp16, K fp32 additions, and above 64 rows the rounding of
+    s (q - z) to fp16."""
+    from fastllm_py.kernels import marlin
+
+    torch = torch_gpu
+    rng = np.random.default_rng(M * 7 + K + N)
+    W = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    pay, w_hat, _ = _prep(torch, W, 128)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a = torch.randn(M, K, generator=g, device="cuda").half()
+    buf = torch.full(((M + 1) * N,), float("nan"), dtype=torch.float16, device="cuda")
+    out = marlin.gemm_fast(a, pay["qweight"], pay["scales"], pay["zeros"], N, K, out=buf[:M * N].view(M, N))
+    torch.cuda.synchronize()
+    assert torch.isnan(buf[M * N:]).all()
+    w = torch.from_numpy(w_hat).cuda().double()
+    ref, mag = a.double() @ w.T, a.double().abs() @ w.abs().T
+    bound = 2.0 ** -11 * ref.abs() + (K * 2.0 ** -24 + (2.0 ** -11 if M > 64 else 0.0)) * mag + 2.0 ** -24
+    assert ((out.double() - ref).abs() <= bound).all()
+    again = marlin.gemm_fast(a, pay["qweight"], pay["scales"], pay["zeros"], N, K)
+    assert torch.equal(out, again)  # fixed order of every sum
+
+
 @pytest.mark.parametrize("M", [1, 16, 256])
 def test_stream_entry_bit_identical(torch_gpu, M):
     # reference tests/test_native_kernels.py:132-154
