@@ -1769,6 +1769,8 @@ struct MoeArgs {
     // token in one fixed order, instead of fp32 atomics into y
     int det, nq;
     float* part;
+    // grouped kernels: units of this launch (see mg_unit)
+    int st_sh, st_r, nch_sh, nch_r;
 };
 
 // Fused routing of the one token (T == 1) in a routed gate/up workgroup:
@@ -2790,15 +2792,15 @@ __global__ __launch_bounds__(256) void moe_combine_k(MoeArgs a) {
 // ------------------------------------------- grouped MoE GEMM (prefill)
 // The two fused-MoE kernels for T > 16 tokens: per list slot a grouped GEMM
 // over the slot's entries, in chunks of 64 rows (4 m-tiles).
-//   PHASE 0 (gate/up): one workgroup per (slot, 128 intermediate columns);
+//   PHASE 0 (gate/up): a workgroup takes 128 intermediate columns of a slot;
 //     wave w computes gate tile 8 strip + w and up tile 8 strip + w over all
 //     of hidden, so h = silu(g) * u * w_entry is formed in registers and
 //     stored fp16 to inter_buf (no cross-wave reduction: waves split N).
 //     Its token rows come from xh, the fp16 copy of x made by x_to_f16_k.
-//   PHASE 1 (down): one workgroup per (slot, 256 hidden columns); wave w
+//   PHASE 1 (down): a workgroup takes 256 hidden columns of a slot; wave w
 //     computes tiles 16 strip + 2 w, + 1 over the slot's inter_buf rows and
 //     adds them into y[token] with fp32 atomics, like the decode kernel.
-// Slot indices >= max_slots are the shared expert (rows max_entries + t,
+// The shared expert is one more slot (rows max_entries + t,
 // tokens t = 0..T-1, coefficient scoef[t] or 1).
 // Every main-loop load goes global -> LDS (lds_copy: buffer_load ... lds
 // from inline asm, see common.cuh), kMgAhead blocks ahead, into a ring of
@@ -2841,6 +2843,34 @@ __global__ void x_to_f16_k(const float* __restrict__ x, uint16_t* __restrict__ x
     }
 }
 
+// A grouped launch's units, one workgroup each: (64-row chunk, column strip)
+// of the shared expert, then (slot, chunk, strip) of the routed ones.  The
+// shared expert has T rows, so its chunks are spread over st_sh x nch_sh
+// workgroups: as one workgroup's loop over 1000 rows they took 509 / 1128 us
+// (gate/up / down, FP8, 60 experts top 4 + shared 5632) where the whole
+// launch now takes 211 / 120.  A slot's rows are known only on the
+// device: it gets nch_r workgroups per strip, workgroup c taking chunks c,
+// c + nch_r, ... (moe_launch_grouped picks nch_r by the mean).
+// The shared units come first: the down projection's have the longest K.
+// Units are XCD-grouped (the hardware deals workgroup L to XCD L % 8, so
+// with the count a multiple of 8 XCD x takes a contiguous run, whose strips
+// share the activation rows in one L2), the two lists each by itself so that
+// every XCD gets its share of the long ones.
+struct MgUnit {
+    int slot, strip, mc, mstep;  // slot < 0: shared expert; chunks mc, mc + mstep, ... (rows)
+};
+FL_DEV MgUnit mg_unit(const MoeArgs& a) {
+    const int ush = a.st_sh * a.nch_sh;
+    const bool sh = (int)blockIdx.x < ush;
+    const int n = sh ? ush : (int)gridDim.x - ush, lin = sh ? (int)blockIdx.x : (int)blockIdx.x - ush;
+    const int u = (n & 7) ? lin : (lin & 7) * (n >> 3) + (lin >> 3);
+    if (sh) return MgUnit{-1, u % a.st_sh, u / a.st_sh * 64, a.nch_sh * 64};
+    // (a division is tens of scalar operations at a workgroup's start)
+    const int y = u / a.st_r;
+    if (a.nch_r == 1) return MgUnit{y, u - y * a.st_r, 0, 64};
+    return MgUnit{y / a.nch_r, u - y * a.st_r, y % a.nch_r * 64, a.nch_r * 64};
+}
+
 template <int PHASE, bool G128, int FMT = kFmtInt4>
 __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -2858,20 +2888,15 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, kq = lane >> 4;
-    // XCD-grouped units, as in moe_gemm_rk
-    const int lin = blockIdx.y * gridDim.x + blockIdx.x, units = gridDim.x * gridDim.y;
-    const int unit = (units & 7) ? lin : (lin & 7) * (units >> 3) + (lin >> 3);
-    const int slot = unit / gridDim.x, strip = unit - slot * gridDim.x;
+    const MgUnit un = mg_unit(a);
+    const int slot = un.slot, strip = un.strip;
     if (PHASE == 0) {
         // every workgroup zeroes its share of y for the down phase's atomics
-        const int nwg = gridDim.x * gridDim.y;
-        const int wg = blockIdx.y * gridDim.x + blockIdx.x;
         const int n4 = a.T * a.hidden / 4;
-        for (int i = wg * 64 * NW + threadIdx.x; i < n4; i += nwg * 64 * NW)
+        for (int i = blockIdx.x * 64 * NW + threadIdx.x; i < n4; i += gridDim.x * 64 * NW)
             reinterpret_cast<f32x4*>(a.y)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    const bool is_shared = slot >= a.max_slots;
-    if (is_shared && !a.has_shared) return;
+    const bool is_shared = slot < 0;
     int e = 0, row0, M;
     const MoeExperts* ex;
     if (!is_shared) {
@@ -2890,7 +2915,7 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
     const int K = PHASE == 0 ? a.hidden : inter;
     const int Nrows = PHASE == 0 ? inter : a.hidden;  // output rows of the weight
     const int ncols = PHASE == 0 ? 16 * NW : 32 * NW;  // columns per workgroup
-    if (M <= 0 || strip * ncols >= Nrows) return;
+    if (un.mc >= M || strip * ncols >= Nrows) return;
     const int nkb = K >> 7;
     const int G = K / a.gs;
     const int spb = 128 / a.gs;  // groups per 128-k block
@@ -2933,7 +2958,7 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
     const int zstep = FMT == kFmtFp8 ? 4 : (FMT == kFmtMx4 ? 64 : spb * 64);  // scale bytes per block
     const int g_local = kq * 32 / a.gs;  // this lane's group within a block
 
-    for (int mc = 0; mc < M; mc += 64) {
+    for (int mc = un.mc; mc < M; mc += un.mstep) {
         const int mt_live = (M - mc + 15) >> 4;  // m-tiles holding rows of this chunk
         // A copies f = FPW wave + i of this wave.  FP8 / MXFP4 (ROWA): chunk
         // rows 4 f .. 4 f + 3 (m-tile f / 4), each the row's whole 256 bytes
@@ -3142,12 +3167,10 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
 // wave's copies and retires the stage of block c - 1, which the copies of
 // block c + kMrD (issued after the barrier) overwrite.
 constexpr int kMrD = 3;              // blocks in flight ahead
-// Waves per workgroup and blocks ahead of each launch.  Config 5 (INT4):
-// 8 / 3 for both 111-112 us per layer; four-wave workgroups two blocks ahead
-// (three per CU, 95 / 82 VGPRs) 119 us for down alone, 124 for gate/up
-// alone, 131 for both; three ahead at four waves 129 us.
-constexpr int kMrGuWaves = 8, kMrGuD = 3;  // gate/up: waves (16 columns each), blocks ahead
-constexpr int kMrDnWaves = 8, kMrDnD = 3;  // down: waves (32 columns each), blocks ahead
+// Eight waves three blocks ahead, 512 tokens over 128 experts (INT4): 111-112
+// us per layer; four-wave workgroups two blocks ahead (three per CU, 95 / 82
+// VGPRs) 119 us for down alone, 124 for gate/up alone, 131 for both; three
+// ahead at four waves 129 us.
 
 template <int V>
 struct IntC {
@@ -3166,23 +3189,15 @@ __global__ __launch_bounds__(64 * NW) void moe_gemm_rk(MoeArgs a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, kq = lane >> 4;
-    // XCD-grouped units: the hardware deals workgroup L (linear index) to XCD
-    // L % 8, so with the unit count a multiple of 8 XCD x takes the
-    // contiguous units [x U/8, (x+1) U/8): whole slots, whose strips then
-    // share the slot's activation rows in one L2
-    const int lin = blockIdx.y * gridDim.x + blockIdx.x, units = gridDim.x * gridDim.y;
-    const int unit = (units & 7) ? lin : (lin & 7) * (units >> 3) + (lin >> 3);
-    const int slot = unit / gridDim.x, strip = unit - slot * gridDim.x;
+    const MgUnit un = mg_unit(a);
+    const int slot = un.slot, strip = un.strip;
     if (PHASE == 0) {
         // every workgroup zeroes its share of y for the down phase's atomics
-        const int nwg = gridDim.x * gridDim.y;
-        const int wg = blockIdx.y * gridDim.x + blockIdx.x;
         const int n4 = a.T * a.hidden / 4;
-        for (int i = wg * 64 * NW + threadIdx.x; i < n4; i += nwg * 64 * NW)
+        for (int i = blockIdx.x * 64 * NW + threadIdx.x; i < n4; i += gridDim.x * 64 * NW)
             reinterpret_cast<f32x4*>(a.y)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    const bool is_shared = slot >= a.max_slots;
-    if (is_shared && !a.has_shared) return;
+    const bool is_shared = slot < 0;
     int e = 0, row0, M;
     const MoeExperts* ex;
     if (!is_shared) {
@@ -3199,7 +3214,7 @@ __global__ __launch_bounds__(64 * NW) void moe_gemm_rk(MoeArgs a) {
     const int K = PHASE == 0 ? a.hidden : inter;
     const int Nrows = PHASE == 0 ? inter : a.hidden;
     const int ncols = PHASE == 0 ? 16 * NW : 32 * NW;
-    if (M <= 0 || strip * ncols >= Nrows) return;
+    if (un.mc >= M || strip * ncols >= Nrows) return;
     const int nkb = K >> 7;
     const int G = K / a.gs;
     const int spb = 128 / a.gs;  // groups per 128-k block
@@ -3232,7 +3247,7 @@ __global__ __launch_bounds__(64 * NW) void moe_gemm_rk(MoeArgs a) {
     const i32x4_t rA = raw_rsrc(abase, (uint32_t)arows * astride * 2);
     const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
 
-    for (int mc = 0; mc < M; mc += 64) {
+    for (int mc = un.mc; mc < M; mc += un.mstep) {
         const int mt_live = (M - mc + 15) >> 4;  // m-tiles holding rows of this chunk
         // lane l holds row mc + l's token and combine weight (rows past M
         // repeat row M - 1), read once per chunk and handed out by shuffles
@@ -3636,16 +3651,16 @@ void launch_down_ns(const MoeArgs& a, const MoePlan& p, hipStream_t st) {
 }
 
 template <int FMT, bool G128>
-void launch_grouped_pair(const MoeArgs& a, dim3 gu, dim3 dn, hipStream_t st) {
+void launch_grouped_pair(const MoeArgs& gu, const MoeArgs& dn, hipStream_t st) {
+    const auto grid = [](const MoeArgs& a) { return dim3(a.st_sh * a.nch_sh + a.st_r * a.nch_r * a.max_slots); };
     if constexpr (FMT == kFmtInt4) {
-        constexpr int GW = kMrGuWaves, GD = kMrGuD, DW = kMrDnWaves, DD = kMrDnD;
-        hipLaunchKernelGGL((moe_gemm_rk<0, G128, GW, GD>), dim3(gu.x * kMgWaves / GW, gu.y), dim3(64 * GW),
-                           (size_t)(GD + 1) * kMgABytes, st, a);
-        hipLaunchKernelGGL((moe_gemm_rk<1, G128, DW, DD>), dim3(dn.x * kMgWaves / DW, dn.y), dim3(64 * DW),
-                           (size_t)(DD + 1) * kMgABytes, st, a);
+        hipLaunchKernelGGL((moe_gemm_rk<0, G128>), grid(gu), dim3(64 * kMgWaves), (size_t)(kMrD + 1) * kMgABytes, st,
+                           gu);
+        hipLaunchKernelGGL((moe_gemm_rk<1, G128>), grid(dn), dim3(64 * kMgWaves), (size_t)(kMrD + 1) * kMgABytes, st,
+                           dn);
     } else {
-        hipLaunchKernelGGL((moe_gemm_k<0, G128, FMT>), gu, dim3(64 * kMgWaves), mg_lds(FMT), st, a);
-        hipLaunchKernelGGL((moe_gemm_k<1, G128, FMT>), dn, dim3(64 * kMgWaves), mg_lds(FMT), st, a);
+        hipLaunchKernelGGL((moe_gemm_k<0, G128, FMT>), grid(gu), dim3(64 * kMgWaves), mg_lds(FMT), st, gu);
+        hipLaunchKernelGGL((moe_gemm_k<1, G128, FMT>), grid(dn), dim3(64 * kMgWaves), mg_lds(FMT), st, dn);
     }
 }
 
@@ -3658,17 +3673,24 @@ void moe_launch_grouped(const MoeArgs& a, hipStream_t st) {
     if (!a.xh_ready)
         hipLaunchKernelGGL(x_to_f16_k, dim3((n8 + 255) / 256 < 1024 ? (n8 + 255) / 256 : 1024), dim3(256), 0,
                            st, a.x, const_cast<uint16_t*>(a.xh), n8);
-    const int slots = a.max_slots + (a.has_shared ? 1 : 0);
-    const int inter_max = a.routed.inter > a.shared.inter ? a.routed.inter : a.shared.inter;
-    const dim3 gu(inter_max / (16 * kMgWaves), slots), dn(a.hidden / (32 * kMgWaves), slots);
+    MoeArgs gu = a, dn = a;
+    gu.st_r = a.routed.inter / (16 * kMgWaves);
+    gu.st_sh = a.has_shared ? a.shared.inter / (16 * kMgWaves) : 0;
+    dn.st_r = a.hidden / (32 * kMgWaves);
+    dn.st_sh = a.has_shared ? dn.st_r : 0;
+    gu.nch_sh = dn.nch_sh = a.has_shared ? (a.T + 63) / 64 : 0;
+    // chunk workgroups per slot: for 1.5 times the mean rows of a slot (they
+    // loop over what is left; a token is at most once in a slot's list)
+    const long rows = a.max_entries * 3l / 2 / a.max_slots;
+    gu.nch_r = dn.nch_r = ((rows < a.T ? (int)rows : a.T) + 63) / 64;
     if (a.fmt == kFmtFp8)
-        launch_grouped_pair<kFmtFp8, true>(a, gu, dn, st);
+        launch_grouped_pair<kFmtFp8, true>(gu, dn, st);
     else if (a.fmt == kFmtMx4)
-        launch_grouped_pair<kFmtMx4, true>(a, gu, dn, st);
+        launch_grouped_pair<kFmtMx4, true>(gu, dn, st);
     else if (a.gs == 128)
-        launch_grouped_pair<kFmtInt4, true>(a, gu, dn, st);
+        launch_grouped_pair<kFmtInt4, true>(gu, dn, st);
     else
-        launch_grouped_pair<kFmtInt4, false>(a, gu, dn, st);
+        launch_grouped_pair<kFmtInt4, false>(gu, dn, st);
     if (a.det) launch_combine(a, st);
 }
 

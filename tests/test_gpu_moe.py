@@ -760,6 +760,33 @@ def test_fused_moe_prefill(torch_gpu, T, E, K, hidden, inter, sinter, gs, norm):
     assert Q.max_abs_rel(y.cpu().numpy(), ref) < 5e-3
 
 
+@pytest.mark.parametrize("T,sinter,gs", [(400, 256, 128), (193, 128, 32)])
+def test_moe_prefill_skewed(torch_gpu, T, sinter, gs):
+    """One expert holds every token, several times the mean that the launch
+    gives each slot chunks for, and the shared expert's rows spread over
+    chunks of their own (the last one ragged)."""
+    from fastllm_py.kernels import moe_int4
+
+    torch = torch_gpu
+    E, K, hidden, inter = 8, 2, 256, 128
+    rng = np.random.default_rng(1800 + T)
+    st, st_o = _stacked(_experts(rng, E, hidden, inter, 0.05), gs)
+    sh, sh_o = _stacked(_experts(rng, 1, hidden, sinter, 0.05), gs)
+    x = (rng.standard_normal((T, hidden)) * 0.5).astype(np.float32)
+    lg = rng.standard_normal((T, E)).astype(np.float32)
+    lg[:, 3] += 10
+    sl = rng.standard_normal(T).astype(np.float32)
+    o = {}
+    y = moe_int4.moe_route_forward(torch.from_numpy(x).cuda(), torch.from_numpy(lg).cuda(), st, K, E, hidden, inter,
+                                   shared=sh, shared_inter=sinter, shared_logit=torch.from_numpy(sl).cuda(), route=o)
+    torch.cuda.synchronize()
+    ids, w = o["topk_ids"].cpu().numpy(), o["topk_w"].cpu().numpy()
+    assert (ids == 3).any(1).all()
+    ref = OM.moe_ref_grouped(x, OM.dequant_stacked(st_o, gs), ids, w, OM.dequant_stacked(sh_o, gs),
+                             1.0 / (1.0 + np.exp(-sl)))
+    assert Q.max_abs_rel(y.cpu().numpy(), ref) < 5e-3
+
+
 def test_moe_prefill_config5(torch_gpu):
     """BASELINE config 5 (Qwen3-30B-A3B MoE layer at M=512): 128 experts,
     hidden 2048, inter 768, top-8 softmax with renormalisation from fp16

@@ -242,6 +242,32 @@ def test_lowp_moe_prefill_parity(torch_gpu, fmt, T, E, K, hidden, inter, sinter,
     assert Q.max_abs_rel(y2.cpu().numpy(), y.cpu().numpy()) < 1e-6, fmt
 
 
+@pytest.mark.parametrize("fmt", ["fp8", "mxfp4"])
+@pytest.mark.parametrize("T,sinter", [(400, 256), (193, 128)])
+def test_lowp_moe_prefill_skewed(torch_gpu, fmt, T, sinter):
+    """One expert holds every token, several times the mean that the launch
+    gives each slot chunks for, and the shared expert's rows spread over
+    chunks of their own (the last one ragged)."""
+    from fastllm_py.kernels import moe_int4
+
+    torch = torch_gpu
+    E, K, hidden, inter = 8, 2, 256, 128
+    rng = np.random.default_rng(1700 + T)
+    st, deq, sh, sdeq = _layer(rng, fmt, E, hidden, inter, sinter)
+    x = torch.from_numpy((rng.standard_normal((T, hidden)) * 0.5).astype(np.float32)).cuda()
+    lg = rng.standard_normal((T, E)).astype(np.float32)
+    lg[:, 3] += 10
+    sl = torch.from_numpy(rng.standard_normal(T).astype(np.float32)).cuda()
+    o = {}
+    y = moe_int4.moe_route_forward(x, torch.from_numpy(lg).cuda(), st, K, E, hidden, inter, shared=sh,
+                                   shared_inter=sinter, shared_logit=sl, route=o)
+    torch.cuda.synchronize()
+    ids, w = o["topk_ids"].cpu().numpy(), o["topk_w"].cpu().numpy()
+    assert (ids == 3).any(1).all()
+    ref = OM.moe_ref_grouped(x.cpu().numpy(), deq, ids, w, sdeq, 1.0 / (1.0 + np.exp(-sl.cpu().numpy())))
+    assert Q.max_abs_rel(y.cpu().numpy(), ref) < TOL
+
+
 def test_lowp_rejects(torch_gpu):
     """A wrong group size or mixed formats are refused before any launch."""
     from fastllm_py import _native
