@@ -62,3 +62,31 @@ __host__ __device__ inline float e4m3_decode_exact(uint8_t b) {
     const float v = e > 0 ? ldexpf(1.0f + (float)m * 0.125f, e - 7) : (float)m * 0.001953125f;
     return (b & 0x80) ? -v : v;
 }
+
+// The 8 e4m3 codes of two words as fp16 / bf16, exactly.
+template <bool BF16>
+FL_DEV u32x4 fp8x8_to_16(uint32_t w0, uint32_t w1) {
+    if (BF16) {
+        return u32x4{bitcast<uint32_t>(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, false)),
+                     bitcast<uint32_t>(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, true)),
+                     bitcast<uint32_t>(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.0f, false)),
+                     bitcast<uint32_t>(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.0f, true))};
+    } else {
+        return u32x4{bitcast<uint32_t>(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w0, 1.0f, false)),
+                     bitcast<uint32_t>(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w0, 1.0f, true)),
+                     bitcast<uint32_t>(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w1, 1.0f, false)),
+                     bitcast<uint32_t>(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w1, 1.0f, true))};
+    }
+}
+
+// fp32 <-> fp16 / bf16 activations
+template <bool BF16>
+FL_DEV uint16_t f32_to_act(float v) {
+    if (BF16) return bitcast<uint16_t>((__bf16)v);
+    return bitcast<uint16_t>((f16)v);
+}
+template <bool BF16>
+FL_DEV float act_to_f32(uint16_t v) {
+    if (BF16) return (float)bitcast<__bf16>(v);
+    return (float)bitcast<f16>(v);
+}

@@ -185,6 +185,42 @@ def test_fp8_block_gemm_prefill(torch_gpu, M, N, K, bf16):
     assert Q.max_abs_rel(out.float().cpu().numpy(), ref) < TOL
 
 
+# every tile shape of the kernel above 16 rows, at ragged rows and columns, K
+# ending in a 64-wide block and fewer k blocks than k groups
+@pytest.mark.parametrize("M,N,K,bf16", [
+    (17, 40, 128, True), (33, 1000, 320, False), (64, 2048, 1024, True),  # 32 x 32, six k groups
+    (20, 10900, 1984, True), (32, 10900, 2048, False),                    # 32 x 64
+    (40, 10900, 192, False), (64, 10944, 1088, True),                     # 64 x 64, three k groups
+    (65, 100, 192, True), (129, 1000, 320, False),                        # 64 x 64, two k groups
+    (100, 10900, 192, True), (66, 10944, 1024, False),                    # 64 x 128
+    (1000, 4090, 192, False), (961, 4096, 640, True),                     # 64 x 256
+    (1000, 6000, 192, True), (900, 6144, 640, False),                     # 128 x 256
+])
+def test_fp8_block_gemm_tile_shapes(torch_gpu, M, N, K, bf16):
+    """Against the float64 product of the same codes and scales.  Bound: the
+    result's rounding to 16 bits and K fp32 additions (the codes are exact)."""
+    from fastllm_py.kernels import fp8
+
+    torch = torch_gpu
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    dt = torch.bfloat16 if bf16 else torch.float16
+    x = torch.randn(M, K, generator=g, device="cuda").to(dt)
+    bias = torch.randn(N, generator=g, device="cuda").to(dt)
+    q = torch.randn(N, K, generator=g, device="cuda").mul(60).to(torch.float8_e4m3fn)
+    sc = torch.rand(-(-N // 128), -(-K // 128), generator=g, device="cuda") * 1e-3
+    buf = torch.full(((M + 1) * N,), float("nan"), dtype=dt, device="cuda")
+    out = fp8.fp8_gemv_block(x, q.view(torch.uint8), sc, bias=bias, out=buf[:M * N].view(M, N))
+    torch.cuda.synchronize()
+    assert torch.isnan(buf[M * N:]).all()
+    w = q.double() * sc.double().repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)[:, :K]
+    ref = x.double() @ w.T + bias.double()
+    mag = x.double().abs() @ w.abs().T + bias.double().abs()
+    eps = 2.0 ** -8 if bf16 else 2.0 ** -11
+    assert ((out.double() - ref).abs() <= eps * ref.abs() + (K + 8) * 2.0 ** -24 * mag + 2.0 ** -24).all()
+    again = fp8.fp8_gemv_block(x, q.view(torch.uint8), sc, bias=bias)
+    assert torch.equal(out, again)  # fixed order of every sum
+
+
 def test_fp8_block_gemm_split_k(torch_gpu):
     """Split-K of the prefill GEMM (grids under 256 tiles): within the
     oracle's tolerance, bit-identical on a repeat (partials summed in split
