@@ -53,23 +53,45 @@ def swiglu(gate, up, out=None, stream=None):
     rows may be strided views (e.g. the two halves of a gate/up output).
     ``out``: optional contiguous fp16 tensor of the same shape."""
     t = nat.torch()
-    g, u = nat.to_device(gate), nat.to_device(up)
+    g, u = _device_view(gate), _device_view(up)
     if g.dtype != t.float16 or u.dtype != t.float16:
         raise TypeError("swiglu: gate and up must be fp16")
     if g.shape != u.shape:
         raise ValueError(f"swiglu: gate {tuple(g.shape)} and up {tuple(u.shape)} differ")
     cols = g.shape[-1]
-    g2, u2 = g.reshape(-1, cols), u.reshape(-1, cols)
-    for v in (g2, u2):
-        if v.stride(-1) != 1:
-            raise ValueError("swiglu: rows must be contiguous")
-    rows = g2.shape[0]
     if out is None:
         out = t.empty(g.shape, dtype=t.float16, device=g.device)
     else:
         nat.check_out(out, g.numel(), (t.float16,), g.device)
+    g2, u2 = _rows(g, cols, out), _rows(u, cols, out)
+    rows = g2.shape[0]
     hs = nat.stream_handle(stream) if stream is not None else nat.current_stream_handle()
     rc = nat.lib().fastllm_swiglu(nat.ptr(g2), nat.ptr(u2), nat.ptr(out), rows, cols,
                                   g2.stride(0), u2.stride(0), cols, hs)
     nat.check_rc(rc, "fastllm_swiglu")
     return out
+
+
+def _device_view(x):
+    """x on the GPU, as it lies there when it is a device tensor already."""
+    return x if nat.is_tensor(x) and x.is_cuda else nat.to_device(x)
+
+
+def _rows(v, cols, out):
+    """v (..., cols) as the (rows, cols) rows that the kernel reads: v's own
+    memory when its rows are evenly spaced, do not overlap and hold their
+    columns side by side (the halves of a gate/up output), else a contiguous
+    copy.  A spaced v that shares memory with ``out`` is copied too: the kernel
+    would store rows over others not yet read."""
+    if v.is_contiguous():
+        return v.reshape(-1, cols)
+    v2 = v.reshape(-1, cols)
+    rows, step = v2.shape[0], v2.stride(0)
+    if v2.stride(1) != 1 or (rows > 1 and not cols <= step < 1 << 31):
+        return v2.contiguous()
+    if rows == 1:
+        return v2.as_strided((1, cols), (cols, 1))
+    a, o = v2.data_ptr(), out.data_ptr()
+    if a < o + 2 * out.numel() and o < a + 2 * ((rows - 1) * step + cols):
+        return v2.contiguous()
+    return v2

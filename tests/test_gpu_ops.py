@@ -40,6 +40,27 @@ def test_add_rmsnorm_matches_oracle(torch_gpu, rows, dim, xt, dt, wt):
     np.testing.assert_allclose(h.float().cpu().numpy(), ref, rtol=1e-3, atol=2e-3)
 
 
+@pytest.mark.parametrize("rows,cols,gap,off", [(1, 1, 0, 0), (3, 7, 0, 0), (5, 768, 0, 0), (2, 2056, 8, 0),
+                                               (4, 1024, 3, 0), (4, 1024, 8, 1), (70000, 8, 0, 0)])
+def test_swiglu_rows(torch_gpu, rows, cols, gap, off):
+    """Both widths of the kernel (8 halves per thread, and one where the rows
+    or the pointers are off 16 bytes) on spaced rows, against float64; bound:
+    the fp16 result and three fp32 roundings with expf's two ulps."""
+    from fastllm_py.kernels import ops
+
+    torch = torch_gpu
+    g = torch.Generator(device="cuda").manual_seed(rows + cols)
+    ld = 2 * cols + gap
+    buf = (torch.randn(rows * ld + off, generator=g, device="cuda") * 3).half()
+    gu = buf[off:].view(rows, ld)
+    out = ops.swiglu(gu[:, :cols], gu[:, cols:2 * cols])
+    torch.cuda.synchronize()
+    a, b = gu[:, :cols].double(), gu[:, cols:2 * cols].double()
+    ref = a / (1 + torch.exp(-a)) * b
+    assert out.shape == (rows, cols)
+    assert ((out.double() - ref).abs() <= (2.0 ** -11 + 2.0 ** -20) * ref.abs() + 2.0 ** -24).all()
+
+
 def test_add_rmsnorm_rejects(torch_gpu):
     from fastllm_py import _native as nat
 
