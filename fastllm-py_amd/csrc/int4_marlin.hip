@@ -835,7 +835,11 @@ struct CsBlk {
     uint16_t s;
 };
 
-template <int MR>
+// SWI: gate/up with the SwiGLU epilogue, as int4_gemv_nb's -- waves 2 i and
+// 2 i + 1 take gate tile s and up tile I/16 + s; the up wave hands its fp16
+// sums over through LDS and C is H, M x I (gate_up 24576 x 4096, M = 13:
+// 15.3 us against 18.5 for the split-k kernel with the epilogue).
+template <int MR, bool SWI>
 __global__ __launch_bounds__(64 * kCsWaves) void int4_gemv_cs(const f16* __restrict__ A,
                                                               const uint32_t* __restrict__ Wq,
                                                               const uint16_t* __restrict__ S,
@@ -848,7 +852,7 @@ __global__ __launch_bounds__(64 * kCsWaves) void int4_gemv_cs(const f16* __restr
     const int nkb = K >> 7, ntiles = N >> 4, zwords = N >> 3;
     const int tb = xcd_block() * kCsWaves + wave;  // this wave's n-tile
     const bool tlive = tb < ntiles;
-    const int nt = tlive ? tb : ntiles - 1;
+    const int nt = !tlive ? ntiles - 1 : SWI ? (tb & 1) * (ntiles >> 1) + (tb >> 1) : tb;
     // activation rows into LDS: one copy = 4 rows x 256 B of one block
     {
         const i32x4_t rA = raw_rsrc(A, (uint32_t)M * (uint32_t)K * 2u);
@@ -932,13 +936,47 @@ __global__ __launch_bounds__(64 * kCsWaves) void int4_gemv_cs(const f16* __restr
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    if (tlive) {
+    if constexpr (SWI) {
+        // after the activation rows, which other waves may still read
+        float* xch = reinterpret_cast<float*>(smem + (size_t)nkb * MR * 256) + (wave >> 1) * 256 + lane;
+        if (wave & 1) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) xch[64 * e] = (float)(f16)acc[e];
+        }
+        lds_barrier();
+        if (!(wave & 1) && tlive) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int m = 4 * kq + e;
+                const float g = (float)(f16)acc[e], u = xch[64 * e];
+                if (m < M) C[(size_t)m * (N >> 1) + nt * 16 + col] = (f16)(g / (1.0f + expf(-g)) * u);
+            }
+        }
+    } else if (tlive) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int m = 4 * kq + e;
             if (m < M) C[(size_t)m * N + nt * 16 + col] = (f16)acc[e];
         }
     }
+}
+
+// Whether a shape takes int4_gemv_cs, and its launch.
+bool gemv_cs_ok(int M, int N, int K, bool g32) {
+    return !g32 && M > 4 && M <= 16 && K % 128 == 0 && N / 16 >= kCsMinTiles && (size_t)N * K / 2 < (1ull << 31) &&
+           (size_t)(K / 128) * (M > 8 ? 16 : 8) * 256 <= 128 * 1024;
+}
+template <bool SWI>
+hipError_t launch_gemv_cs(const f16* A, const uint32_t* Wq, const uint16_t* S, const uint32_t* Z, f16* C, int M, int N,
+                          int K, hipStream_t stream) {
+    const int mr = M > 8 ? 16 : 8;
+    const size_t lds = (size_t)(K / 128) * mr * 256 + (SWI ? kCsWaves / 2 * 1024 : 0);
+    const dim3 grid((N / 16 + kCsWaves - 1) / kCsWaves), block(64 * kCsWaves);
+    if (mr == 16)
+        hipLaunchKernelGGL((int4_gemv_cs<16, SWI>), grid, block, lds, stream, A, Wq, S, Z, C, M, N, K);
+    else
+        hipLaunchKernelGGL((int4_gemv_cs<8, SWI>), grid, block, lds, stream, A, Wq, S, Z, C, M, N, K);
+    return hipGetLastError();
 }
 
 // Prefill-shaped GEMM of group-32 weights (M > 64, K % 128 == 0) on the
@@ -1487,20 +1525,9 @@ bool int4_marlin_abi_gemm(const void* a, const uint32_t* q, const void* scales,
     if (M > 16)
         return int4_gemm_large_m(A, q, static_cast<const f16*>(scales), zeros, Cp, M, N, K, g32,
                                  stream);
-    if (!forced && !g32 && M > 4 && K % 128 == 0 && N / 16 >= kCsMinTiles && (size_t)N * K / 2 < (1ull << 31)) {
-        // wide output, 5..16 rows: the column-split GEMV, all rows in LDS
-        const int mr = M > 8 ? 16 : 8;
-        const size_t lds = (size_t)(K / 128) * mr * 256;
-        if (lds <= 128 * 1024) {
-            const dim3 grid((N / 16 + kCsWaves - 1) / kCsWaves), block(64 * kCsWaves);
-            const uint16_t* S = static_cast<const uint16_t*>(scales);
-            if (mr == 16)
-                hipLaunchKernelGGL(int4_gemv_cs<16>, grid, block, lds, stream, A, q, S, zeros, Cp, M, N, K);
-            else
-                hipLaunchKernelGGL(int4_gemv_cs<8>, grid, block, lds, stream, A, q, S, zeros, Cp, M, N, K);
-            return report(hipGetLastError(), "FastllmCudaMarlinHalfInt4Gemm");
-        }
-    }
+    if (!forced && gemv_cs_ok(M, N, K, g32))  // wide output, 5..16 rows: all rows in LDS
+        return report(launch_gemv_cs<false>(A, q, static_cast<const uint16_t*>(scales), zeros, Cp, M, N, K, stream),
+                      "FastllmCudaMarlinHalfInt4Gemm");
     GemvCfg cfg = forced ? *forced : default_gemv_cfg(M, N, K, g32, ws != nullptr);
     if (cfg.split > 1 && (!ws || !fl_aligned(ws, 256) || N / 16 > kSplitStrips ||
                           ws_bytes < splitk_ws_bytes(M, N, cfg.split))) {
@@ -1789,7 +1816,9 @@ int fastllm_int4_gemm_swiglu(const void* a, const uint32_t* b_q_weight, const vo
     const uint16_t* S = static_cast<const uint16_t*>(b_scales);
     f16* H = static_cast<f16*>(h);
     const hipError_t e =
-        group_size == 32
+        gemv_cs_ok(size_m, size_n, size_k, group_size == 32)
+            ? launch_gemv_cs<true>(A, b_q_weight, S, b_zeros, H, size_m, size_n, size_k, (hipStream_t)stream)
+        : group_size == 32
             ? dispatch_swiglu<true>(A, b_q_weight, S, b_zeros, H, size_m, size_n, size_k, (hipStream_t)stream)
             : dispatch_swiglu<false>(A, b_q_weight, S, b_zeros, H, size_m, size_n, size_k, (hipStream_t)stream);
     if (e == hipErrorInvalidValue) return 1;  // shape beyond the fused kernel (see dispatch_swiglu)

@@ -467,6 +467,31 @@ def test_gemm_swiglu(torch_gpu, M, I, K, gs):
     assert Q.max_abs_rel(got, rg / (1.0 + np.exp(-rg)) * ru) < TOL
 
 
+@pytest.mark.parametrize("M,I,K", [(5, 8192, 128), (8, 8256, 640), (9, 8192, 256), (13, 8256, 4096), (16, 8192, 1152)])
+def test_gemm_swiglu_column_split(torch_gpu, M, I, K):
+    """The wide gate/up kernel's SwiGLU epilogue against its plain form
+    followed by swiglu: the same fp16 sums g and u, then the same fp32
+    expression, whose last multiplication the compiler may join with the
+    conversion to fp16 (one rounding instead of two).  Bound: one spacing of
+    the fp16 result (2^-10 of it, 2^-24 where it is subnormal)."""
+    from fastllm_py.kernels import marlin, ops
+
+    torch = torch_gpu
+    rng = np.random.default_rng(9100 + M + I + K)
+    W = (rng.standard_normal((2 * I, K)) * 0.05).astype(np.float32)
+    pay, _, _ = _prep(torch, W, 128)
+    a = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float16)).cuda()
+    args = (pay["qweight"], pay["scales"], pay["zeros"], 2 * I, K)
+    buf = torch.full(((M + 1) * I,), float("nan"), dtype=torch.float16, device="cuda")
+    h = marlin.gemm_swiglu(a, *args, out=buf[:M * I].view(M, I))
+    gu = marlin.gemm_fast(a, *args, workspace=torch.zeros(1, dtype=torch.int32, device="cuda"))  # no split workspace
+    torch.cuda.synchronize()
+    assert torch.isnan(buf[M * I:]).all()
+    ref = ops.swiglu(gu[:, :I], gu[:, I:]).double()
+    assert ((h.double() - ref).abs() <= 2.0 ** -10 * ref.abs() + 2.0 ** -24).all()
+    assert (h.double() == ref).double().mean() > 0.99
+
+
 def test_gemm_swiglu_rejects(torch_gpu):
     from fastllm_py import _native
 
