@@ -1770,7 +1770,7 @@ struct MoeArgs {
     int det, nq;
     float* part;
     // grouped kernels: units of this launch (see mg_unit)
-    int st_sh, st_r, nch_sh, nch_r;
+    int st_sh, st_r, nch_sh, nch_r, kp_sh;
 };
 
 // Fused routing of the one token (T == 1) in a routed gate/up workgroup:
@@ -2851,24 +2851,36 @@ __global__ void x_to_f16_k(const float* __restrict__ x, uint16_t* __restrict__ x
 // launch now takes 211 / 120.  A slot's rows are known only on the
 // device: it gets nch_r workgroups per strip, workgroup c taking chunks c,
 // c + nch_r, ... (moe_launch_grouped picks nch_r by the mean).
-// The shared units come first: the down projection's have the longest K.
+// The shared units come first, the row chunks of one strip side by side: they
+// share its weights.  The down projection's shared K may be several times a
+// routed expert's, and its units would be the launch's longest chain (5632
+// against 1408: 58 us at T = 64 whatever the rest took), so it is cut into
+// kp_sh pieces that each add to y (not with the deterministic combine, whose
+// term rows hold one piece).
 // Units are XCD-grouped (the hardware deals workgroup L to XCD L % 8, so
 // with the count a multiple of 8 XCD x takes a contiguous run, whose strips
 // share the activation rows in one L2), the two lists each by itself so that
 // every XCD gets its share of the long ones.
 struct MgUnit {
     int slot, strip, mc, mstep;  // slot < 0: shared expert; chunks mc, mc + mstep, ... (rows)
+    int kb0, kbn;                // its K piece: blocks kb0 .. kb0 + kbn - 1 (kbn < 0: all)
 };
 FL_DEV MgUnit mg_unit(const MoeArgs& a) {
-    const int ush = a.st_sh * a.nch_sh;
+    const int ush = a.st_sh * a.nch_sh * a.kp_sh;
     const bool sh = (int)blockIdx.x < ush;
     const int n = sh ? ush : (int)gridDim.x - ush, lin = sh ? (int)blockIdx.x : (int)blockIdx.x - ush;
     const int u = (n & 7) ? lin : (lin & 7) * (n >> 3) + (lin >> 3);
-    if (sh) return MgUnit{-1, u % a.st_sh, u / a.st_sh * 64, a.nch_sh * 64};
     // (a division is tens of scalar operations at a workgroup's start)
-    const int y = u / a.st_r;
-    if (a.nch_r == 1) return MgUnit{y, u - y * a.st_r, 0, 64};
-    return MgUnit{y / a.nch_r, u - y * a.st_r, y % a.nch_r * 64, a.nch_r * 64};
+    if (sh) {
+        const int y = u / a.nch_sh, mc = (u - y * a.nch_sh) * 64;
+        if (a.kp_sh == 1) return MgUnit{-1, y, mc, a.nch_sh * 64, 0, -1};
+        const int strip = y / a.kp_sh, p = y - strip * a.kp_sh;
+        const int nkb = a.shared.inter >> 7, per = (nkb + a.kp_sh - 1) / a.kp_sh, kb0 = p * per;
+        return MgUnit{-1, strip, mc, a.nch_sh * 64, kb0, clampi(nkb - kb0, 0, per)};
+    }
+    const int y = u / a.st_r, strip = u - y * a.st_r;
+    if (a.nch_r == 1) return MgUnit{y, strip, 0, 64, 0, -1};
+    return MgUnit{y / a.nch_r, strip, y % a.nch_r * 64, a.nch_r * 64, 0, -1};
 }
 
 template <int PHASE, bool G128, int FMT = kFmtInt4>
@@ -2916,7 +2928,8 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
     const int Nrows = PHASE == 0 ? inter : a.hidden;  // output rows of the weight
     const int ncols = PHASE == 0 ? 16 * NW : 32 * NW;  // columns per workgroup
     if (un.mc >= M || strip * ncols >= Nrows) return;
-    const int nkb = K >> 7;
+    const int nkb_all = K >> 7, nkb = un.kbn < 0 ? nkb_all : un.kbn;  // the weight's blocks, this unit's
+    if (nkb <= 0) return;
     const int G = K / a.gs;
     const int spb = 128 / a.gs;  // groups per 128-k block
 
@@ -2936,13 +2949,13 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
             tq = ex->dq;
             tsz = ex->dsz;
         }
-        rq[t] = raw_rsrc(tq + tile * nkb * TB, nkb * TB);
+        rq[t] = raw_rsrc(tq + (tile * nkb_all + un.kb0) * TB, nkb * TB);
         if (FMT == kFmtFp8)  // one fp32 scale per (128-row band, block)
-            rz[t] = raw_rsrc(tsz + (tile >> 3) * nkb, nkb * 4);
+            rz[t] = raw_rsrc(tsz + (tile >> 3) * nkb_all + un.kb0, nkb * 4);
         else if (FMT == kFmtMx4)  // 16 E8M0 words per block
-            rz[t] = raw_rsrc(tsz + tile * nkb * 16, nkb * 64);
+            rz[t] = raw_rsrc(tsz + (tile * nkb_all + un.kb0) * 16, nkb * 64);
         else
-            rz[t] = raw_rsrc(tsz + tile * G * 16, G * 64);
+            rz[t] = raw_rsrc(tsz + (tile * G + un.kb0 * spb) * 16, nkb * spb * 64);
     }
     // A rows: PHASE 0 token rows of xh, PHASE 1 the slot's inter_buf rows
     const uint16_t* abase = PHASE == 0 ? a.xh : a.inter_buf;
@@ -2978,7 +2991,7 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
             int m = mc + r;
             m = m < M ? m : M - 1;
             const int row = PHASE == 0 ? __shfl(ltok, m - mc, 64) : row0 + m;
-            ao[i] = 2u * ((uint32_t)row * astride +
+            ao[i] = 2u * ((uint32_t)row * astride + 128u * un.kb0 +
                           (ROWA ? 8 * ((lane & 15) ^ (r & 15)) : a_koff<FMT>(kq, f & 3)));
         }
         // blocks past the end keep the copy count with lane offsets past
@@ -3215,7 +3228,8 @@ __global__ __launch_bounds__(64 * NW) void moe_gemm_rk(MoeArgs a) {
     const int Nrows = PHASE == 0 ? inter : a.hidden;
     const int ncols = PHASE == 0 ? 16 * NW : 32 * NW;
     if (un.mc >= M || strip * ncols >= Nrows) return;
-    const int nkb = K >> 7;
+    const int nkb_all = K >> 7, nkb = un.kbn < 0 ? nkb_all : un.kbn;  // the weight's blocks, this unit's
+    if (nkb <= 0) return;
     const int G = K / a.gs;
     const int spb = 128 / a.gs;  // groups per 128-k block
 
@@ -3235,8 +3249,8 @@ __global__ __launch_bounds__(64 * NW) void moe_gemm_rk(MoeArgs a) {
             tq = ex->dq;
             tsz = ex->dsz;
         }
-        rq[t] = buf_rsrc(tq + tile * nkb * 1024, (uint32_t)nkb * 1024u);
-        rz[t] = buf_rsrc(tsz + tile * G * 16, (uint32_t)G * 64u);
+        rq[t] = buf_rsrc(tq + (tile * nkb_all + un.kb0) * 1024, (uint32_t)nkb * 1024u);
+        rz[t] = buf_rsrc(tsz + (tile * G + un.kb0 * spb) * 16, (uint32_t)(nkb * spb) * 64u);
     }
     const uint32_t zoff = 4u * (uint32_t)((kq * 32 / a.gs) * 16 + col);  // this lane's word in a block
     const uint32_t zstep = (uint32_t)spb * 64u;                           // scale bytes per block
@@ -3262,7 +3276,7 @@ __global__ __launch_bounds__(64 * NW) void moe_gemm_rk(MoeArgs a) {
             const int f = wave * FPW + i;
             const int r = 16 * (f >> 2) + col;  // chunk row
             const int row = PHASE == 0 ? __shfl(ltok, r, 64) : row0 + (mc + r < M ? mc + r : M - 1);
-            ao[i] = 2u * ((uint32_t)row * astride + a_koff<kFmtInt4>(kq, f & 3));
+            ao[i] = 2u * ((uint32_t)row * astride + 128u * un.kb0 + a_koff<kFmtInt4>(kq, f & 3));
         }
         // block b: activation copies into stage b % NS, then the wave's weight
         // and scale loads into r.  Blocks past the end keep the weight and
@@ -3374,6 +3388,248 @@ __global__ __launch_bounds__(64 * NW) void moe_gemm_rk(MoeArgs a) {
                 }
             }
         asm volatile("s_barrier" ::: "memory");  // the chunk's LDS is reused by the next chunk
+    }
+}
+
+// Grouped MoE GEMM of FP8 experts on 32x32x16 MFMAs: the units, chunks and
+// epilogues of moe_gemm_k with four waves of 64 columns (gate/up: 32 gate and
+// the same 32 up columns; down: 64).
+//   * A fragment of 32 rows read from LDS feeds 64 columns, four times those of
+//     a 16-column wave, and the chunk's rows count in steps of 32.
+//   * Weights go to registers one block ahead (each wave's own, whole KB
+//     loads); one v_permlane16_swap of a word of two neighbouring tiles makes
+//     the operands of 32 columns: lane (lc, hi) then holds column lc and, from
+//     words 2 j, 2 j + 1, k 8 (4 h + j + 8 hi) .. + 7 for the swap's results
+//     h = 0, 1.
+//   * Activations: two LDS stages of 64 whole rows (16-byte chunks of row r
+//     XOR-swizzled by r % 16), copied one block ahead.
+//   * The codes are exact and the block's fp32 partial takes the block scale.
+// Two workgroups per CU (32 KB of LDS, 256 VGPRs).  Gate/up / down, FP8, 60
+// experts top 4 + shared 5632, hidden 2048: T = 1000 208 / 119 us with all
+// operands through LDS and 16x16x32 MFMAs (moe_gemm_k) -> 154 / 90,
+// T = 64 81 / 76 -> 75 / 68 (before the shared K pieces); 128 experts top 8, T = 512 87 / 66 -> 82 / 57.
+// The same form for INT4 was no faster than moe_gemm_rk (T = 512 65 / 46
+// against 62 / 43 us, T = 1000 165 / 86 against 164 / 87).
+constexpr int kMwWaves = 4;
+constexpr size_t kMwLds = 2 * kMgABytes;
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+template <int PHASE>
+__global__ __launch_bounds__(64 * kMwWaves, 2) void moe_gemm_wide(MoeArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int NW = kMwWaves, TB = 2048;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lc = lane & 31, hi = lane >> 5;
+    const MgUnit un = mg_unit(a);
+    const int slot = un.slot, strip = un.strip;
+    if (PHASE == 0) {
+        // every workgroup zeroes its share of y for the down phase's atomics
+        const int n4 = a.T * a.hidden / 4;
+        for (int i = blockIdx.x * 64 * NW + threadIdx.x; i < n4; i += gridDim.x * 64 * NW)
+            reinterpret_cast<f32x4*>(a.y)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const bool is_shared = slot < 0;
+    int e = 0, row0, M;
+    const MoeExperts* ex;
+    if (!is_shared) {
+        if (!moe_slot(a, slot, e, row0, M)) return;
+        const int r1 = clampi(__builtin_amdgcn_readfirstlane(a.offsets[slot + 1]), row0, a.max_entries);
+        M = r1 - row0;
+        ex = &a.routed;
+    } else {
+        row0 = a.max_entries;
+        M = a.T;
+        ex = &a.shared;
+    }
+    const int inter = ex->inter;
+    const int K = PHASE == 0 ? a.hidden : inter;
+    const int Nrows = PHASE == 0 ? inter : a.hidden;
+    const int ncols = PHASE == 0 ? 32 * NW : 64 * NW;
+    if (un.mc >= M || strip * ncols >= Nrows) return;
+    const int nkb_all = K >> 7, nkb = un.kbn < 0 ? nkb_all : un.kbn;  // the weight's blocks, this unit's
+    if (nkb <= 0) return;
+
+    // this wave's two tile pairs: 32 weight rows each
+    __amdgpu_buffer_rsrc_t rq[2], rz[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        size_t tile;
+        const uint8_t* tq;
+        const uint32_t* tsz;
+        if (PHASE == 0) {
+            tile = (size_t)e * (inter / 16) + (strip * NW + wave) * 2;
+            tq = u == 0 ? ex->gq : ex->uq;
+            tsz = u == 0 ? ex->gsz : ex->usz;
+        } else {
+            tile = (size_t)e * (a.hidden / 16) + (strip * NW + wave) * 4 + 2 * u;
+            tq = ex->dq;
+            tsz = ex->dsz;
+        }
+        rq[u] = buf_rsrc(tq + (tile * nkb_all + un.kb0) * TB, (uint32_t)(nkb_all + nkb) * TB);
+        // one fp32 scale per (128-row band, block)
+        rz[u] = buf_rsrc(tsz + (tile >> 3) * nkb_all + un.kb0, (uint32_t)nkb * 4u);
+    }
+    const uint16_t* abase = PHASE == 0 ? a.xh : a.inter_buf;
+    const int astride = PHASE == 0 ? a.hidden : a.inter_pad;  // halves
+    const int arows = PHASE == 0 ? a.T : a.max_entries + a.T;
+    const i32x4_t rA = raw_rsrc(abase, (uint32_t)arows * astride * 2);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+
+    for (int mc = un.mc; mc < M; mc += un.mstep) {
+        const int live = M - mc;  // rows of this chunk (64 at most count)
+        // lane l holds row mc + l's token and combine weight (rows past M
+        // repeat row M - 1), read once per chunk and handed out by shuffles
+        const int ml = mc + lane < M ? mc + lane : M - 1;
+        const int ltok = is_shared ? ml : clampi(a.tok[row0 + ml], 0, a.T - 1);
+        const float lw = PHASE != 0 ? 0.0f : (!is_shared ? a.tokw[row0 + ml] : (a.scoef ? a.scoef[ml] : 1.0f));
+        uint32_t ao[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = 4 * (wave * 4 + i) + (lane >> 4);
+            const int row = PHASE == 0 ? __shfl(ltok, r, 64) : row0 + (mc + r < M ? mc + r : M - 1);
+            ao[i] = 2u * ((uint32_t)row * astride + 128u * un.kb0) + 16u * ((lane & 15) ^ (r & 15));
+        }
+        auto copy_a = [&](int kb) {
+            const uint32_t st = lds0 + (uint32_t)(kb & 1) * kMgABytes;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (16 * wave + 4 * i < live) lds_copy(rA, st + (wave * 4 + i) * 1024, ao[i], kb * 256);
+        };
+        // half h of a block's codes, and its scales
+        u32x4 b[4][2];
+        auto load_w = [&](int kb, int h) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                b[t][h] = bitcast<u32x4>(__builtin_amdgcn_raw_buffer_load_b128(
+                    rq[t >> 1], (int)(lane * 16 + h * 1024), (int)(((t & 1) * nkb_all + kb) * TB), 2));
+        };
+        auto load_sz = [&](uint32_t (&sz)[2], int kb) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) sz[u] = __builtin_amdgcn_raw_buffer_load_b32(rz[u], 0, kb * 4, 0);
+        };
+
+        f32x16 acc[2][2];
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[mt][u][i] = 0.f;
+
+        auto run = [&](auto mlc) {
+            constexpr int ML = decltype(mlc)::value;
+            auto read_a = [&](f16x8 (&av)[ML], int kb, int c) {
+                const unsigned char* ab = smem + (size_t)(kb & 1) * kMgABytes + lc * 256;
+#pragma unroll
+                for (int mt = 0; mt < ML; ++mt)
+                    av[mt] = *reinterpret_cast<const f16x8*>(ab + mt * 8192 + 16 * ((c + 8 * hi) ^ (lc & 15)));
+            };
+            // the codes' two KB halves in one register set each: half h of
+            // the next block goes out once this block's half is converted
+            // (a second set of both spilled 102 registers in gate/up)
+            uint32_t sz[2];
+            copy_a(0);
+            load_sz(sz, 0);
+            load_w(0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            load_w(0, 1);
+            for (int kb = 0; kb < nkb; ++kb) {
+                // activations, scales and first halves have landed (the four
+                // loads of the second halves went out last), and the LDS
+                // reads of the stage refilled below are done
+                __builtin_amdgcn_s_waitcnt(4 | (7 << 4));
+                asm volatile("s_barrier" ::: "memory");
+                const float s0 = __uint_as_float(__builtin_amdgcn_readfirstlane(sz[0]));
+                const float s1 = __uint_as_float(__builtin_amdgcn_readfirstlane(sz[1]));
+                const int kn = kb + 1 < nkb ? kb + 1 : kb;  // (the last block loads itself again)
+                if (kb + 1 < nkb) copy_a(kb + 1);
+                f32x16 part[ML][2];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int hh = j >> 1, x = 2 * (j & 1);
+                    f16x8 bv[2][2];  // operands [h][pair]
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const auto r0 = __builtin_amdgcn_permlane16_swap(b[2 * u][hh][x], b[2 * u + 1][hh][x],
+                                                                         false, false);
+                        const auto r1 = __builtin_amdgcn_permlane16_swap(b[2 * u][hh][x + 1],
+                                                                         b[2 * u + 1][hh][x + 1], false, false);
+#pragma unroll
+                        for (int h = 0; h < 2; ++h)
+                            bv[h][u] = bitcast<f16x8>(u32x4{fp8x2_f16(r0[h], false), fp8x2_f16(r0[h], true),
+                                                            fp8x2_f16(r1[h], false), fp8x2_f16(r1[h], true)});
+                    }
+                    if (j == 1 || j == 3) {
+                        asm volatile("" : : "v"(bv[0][0]), "v"(bv[0][1]), "v"(bv[1][0]), "v"(bv[1][1]));
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (j == 1) load_sz(sz, kn);
+                        load_w(kn, hh);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        f16x8 av[ML];
+                        read_a(av, kb, 4 * h + j);
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+#pragma unroll
+                            for (int mt = 0; mt < ML; ++mt) {
+                                const f32x16 z{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
+                                               0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                                part[mt][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                    av[mt], bv[h][u], j == 0 && h == 0 ? z : part[mt][u], 0, 0, 0);
+                            }
+                    }
+                }
+#pragma unroll
+                for (int mt = 0; mt < ML; ++mt)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        acc[mt][0][i] = __builtin_fmaf(s0, part[mt][0][i], acc[mt][0][i]);
+                        acc[mt][1][i] = __builtin_fmaf(s1, part[mt][1][i], acc[mt][1][i]);
+                    }
+            }
+        };
+        if (live > 32)
+            run(IntC<2>{});
+        else
+            run(IntC<1>{});
+
+        // epilogue: lane (lc, hi) holds column lc of each pair, rows mc +
+        // 32 mt + 8 (i / 4) + 4 hi + i % 4
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+            if (32 * mt >= live) break;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int r = 32 * mt + 8 * (i >> 2) + 4 * hi + (i & 3), m = mc + r;
+                // shuffles with every lane active (a lane whose row is past M
+                // may hold the row another lane reads)
+                const float w = __shfl(lw, r, 64);
+                const int tkn = __shfl(ltok, r, 64);
+                if (m >= M) continue;
+                if (PHASE == 0) {
+                    const float g = acc[mt][0][i], up = acc[mt][1][i];
+                    const float h = (g / (1.0f + expf(-g))) * up * w;
+                    a.inter_buf[(size_t)(row0 + m) * a.inter_pad + (strip * NW + wave) * 32 + lc] =
+                        bitcast<uint16_t>((f16)h);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const int cc = (strip * NW + wave) * 64 + u * 32 + lc;
+                        if (a.det)  // the shared slot's rows max_entries + t are piece 0's
+                            a.part[(size_t)(row0 + m) * a.hidden + cc] = acc[mt][u][i];
+                        else
+                            unsafeAtomicAdd(&a.y[(size_t)tkn * a.hidden + cc], acc[mt][u][i]);
+                    }
+                }
+            }
+        }
+        // every wave's LDS reads are done before the next chunk's copies
+        __builtin_amdgcn_s_waitcnt(7 << 4);
+        asm volatile("s_barrier" ::: "memory");
     }
 }
 
@@ -3652,8 +3908,11 @@ void launch_down_ns(const MoeArgs& a, const MoePlan& p, hipStream_t st) {
 
 template <int FMT, bool G128>
 void launch_grouped_pair(const MoeArgs& gu, const MoeArgs& dn, hipStream_t st) {
-    const auto grid = [](const MoeArgs& a) { return dim3(a.st_sh * a.nch_sh + a.st_r * a.nch_r * a.max_slots); };
-    if constexpr (FMT == kFmtInt4) {
+    const auto grid = [](const MoeArgs& a) { return dim3(a.st_sh * a.nch_sh * a.kp_sh + a.st_r * a.nch_r * a.max_slots); };
+    if constexpr (FMT == kFmtFp8) {
+        hipLaunchKernelGGL(moe_gemm_wide<0>, grid(gu), dim3(64 * kMwWaves), kMwLds, st, gu);
+        hipLaunchKernelGGL(moe_gemm_wide<1>, grid(dn), dim3(64 * kMwWaves), kMwLds, st, dn);
+    } else if constexpr (FMT == kFmtInt4) {
         hipLaunchKernelGGL((moe_gemm_rk<0, G128>), grid(gu), dim3(64 * kMgWaves), (size_t)(kMrD + 1) * kMgABytes, st,
                            gu);
         hipLaunchKernelGGL((moe_gemm_rk<1, G128>), grid(dn), dim3(64 * kMgWaves), (size_t)(kMrD + 1) * kMgABytes, st,
@@ -3683,6 +3942,17 @@ void moe_launch_grouped(const MoeArgs& a, hipStream_t st) {
     // loop over what is left; a token is at most once in a slot's list)
     const long rows = a.max_entries * 3l / 2 / a.max_slots;
     gu.nch_r = dn.nch_r = ((rows < a.T ? (int)rows : a.T) + 63) / 64;
+    // K pieces of the shared down units: while they are longer than the
+    // blocks each of 512 workgroups gets of the whole launch (every piece adds
+    // T x hidden atomics: T = 1000 in four pieces 107 us, whole 90; T = 250 / 64
+    // in three / four 51 / 37 us, whole 70 / 68; FP8, shared 5632)
+    gu.kp_sh = dn.kp_sh = 1;
+    if (a.has_shared && !a.det) {
+        const long ks = a.shared.inter / 128, kr = a.routed.inter / 128;
+        const long each = (dn.st_r * (dn.nch_sh * ks + (long)a.max_slots * dn.nch_r * kr) + 511) / 512;
+        const long kp = ks / (each > kr ? each : kr);
+        dn.kp_sh = kp > 1 ? (int)kp : 1;
+    }
     if (a.fmt == kFmtFp8)
         launch_grouped_pair<kFmtFp8, true>(gu, dn, st);
     else if (a.fmt == kFmtMx4)

@@ -760,15 +760,17 @@ def test_fused_moe_prefill(torch_gpu, T, E, K, hidden, inter, sinter, gs, norm):
     assert Q.max_abs_rel(y.cpu().numpy(), ref) < 5e-3
 
 
-@pytest.mark.parametrize("T,sinter,gs", [(400, 256, 128), (193, 128, 32)])
-def test_moe_prefill_skewed(torch_gpu, T, sinter, gs):
+@pytest.mark.parametrize("T,sinter,inter,gs", [(400, 256, 128, 128), (193, 128, 128, 32), (70, 896, 256, 128),
+                                               (70, 896, 256, 32)])
+def test_moe_prefill_skewed(torch_gpu, T, sinter, inter, gs):
     """One expert holds every token, several times the mean that the launch
     gives each slot chunks for, and the shared expert's rows spread over
-    chunks of their own (the last one ragged)."""
+    chunks of their own (the last one ragged); shared 896 beside 256: its
+    down projection's seven blocks of K in pieces of three, three and one."""
     from fastllm_py.kernels import moe_int4
 
     torch = torch_gpu
-    E, K, hidden, inter = 8, 2, 256, 128
+    E, K, hidden = 8, 2, 256
     rng = np.random.default_rng(1800 + T)
     st, st_o = _stacked(_experts(rng, E, hidden, inter, 0.05), gs)
     sh, sh_o = _stacked(_experts(rng, 1, hidden, sinter, 0.05), gs)

@@ -243,15 +243,16 @@ def test_lowp_moe_prefill_parity(torch_gpu, fmt, T, E, K, hidden, inter, sinter,
 
 
 @pytest.mark.parametrize("fmt", ["fp8", "mxfp4"])
-@pytest.mark.parametrize("T,sinter", [(400, 256), (193, 128)])
-def test_lowp_moe_prefill_skewed(torch_gpu, fmt, T, sinter):
+@pytest.mark.parametrize("T,sinter,inter", [(400, 256, 128), (193, 128, 128), (70, 896, 256)])
+def test_lowp_moe_prefill_skewed(torch_gpu, fmt, T, sinter, inter):
     """One expert holds every token, several times the mean that the launch
     gives each slot chunks for, and the shared expert's rows spread over
-    chunks of their own (the last one ragged)."""
+    chunks of their own (the last one ragged); shared 896 beside 256: its
+    down projection's seven blocks of K in pieces of three, three and one."""
     from fastllm_py.kernels import moe_int4
 
     torch = torch_gpu
-    E, K, hidden, inter = 8, 2, 256, 128
+    E, K, hidden = 8, 2, 256
     rng = np.random.default_rng(1700 + T)
     st, deq, sh, sdeq = _layer(rng, fmt, E, hidden, inter, sinter)
     x = torch.from_numpy((rng.standard_normal((T, hidden)) * 0.5).astype(np.float32)).cuda()
