@@ -280,15 +280,28 @@ __global__ __launch_bounds__(1024) void int4_tile_mm(
 // (fastllm_py/kernels/ops.py:157-163).  C is then H, M x I.
 // AM 4 (M = 1): the activation row is add_rmsnorm's output, formed in the
 // prologue from the residual x (fp32), the branch output d (fp16) and the
-// norm weight w (fp16): v = x + d, h = fp16((v * inv) * w) with
-// inv = 1 / sqrt(sum(v^2) / K + eps) (reference: graph_decode.py:300-322).
+// norm weight w (fp16): v = x + d, h = (v * w) * inv with
+// inv = 1 / sqrt(sum(v^2) / K + eps) (reference: graph_decode.py:300-322);
+// fp16(v * w) up to a power of two feeds the MFMAs and inv their result.
 struct NormArgs {
     const float* x;
     const uint16_t* d;
     const uint16_t* w;
     float* xnew;  // x + d, stored by workgroup 0
     float eps;
+    double rk = 0.0;  // 1 / K
 };
+
+// 1 / sqrt(tot / K + eps) rounded once to float, on the way to the last store:
+// a double Newton step from the hardware's float estimate (error below
+// 2^-44) instead of a double square root and two divisions.
+FL_DEV float inv_rms(float tot, double rk, float eps) {
+    const double m = __builtin_fma((double)tot, rk, (double)eps);
+    const float mf = (float)m;
+    if (!(mf > 1e-30f && mf < 1e30f)) return (float)(1.0 / sqrt(m));  // zero, overflow, NaN
+    const double r = (double)__builtin_amdgcn_rsqf(mf);
+    return (float)(r * __builtin_fma(-0.5 * m * r, r, 1.5));
+}
 
 // Split-K (gridDim.y > 1, plain GEMV with register activations only): split
 // s of S covers full blocks [s * nb_s, (s + 1) * nb_s); each split stores its
@@ -557,66 +570,70 @@ __device__ __forceinline__ void int4_gemv_body(const f16* __restrict__ A, const 
         constexpr int WL = NB * (T * (1 + SPB) + (ZSHARE ? 1 : T) * SPB);
         wait_vmcnt<(WL < 63 ? WL : 63)>();
     }
+    // AM 4: per wave the sum of v^2 and the exponent of its h (16 of each)
+    float* npart = reinterpret_cast<float*>(smem + abytes + (size_t)nwaves * T * 1024);
+    int* nexp = reinterpret_cast<int*>(npart + 16);
     if (AM == 4) {
-        // add_rmsnorm of the one row: sum of v^2 over this wave's live
-        // blocks (lane l: elements 2l, 2l + 1), the waves' partials summed in
-        // wave order through LDS (an LDS-only barrier: the weights stay in
-        // flight), then h of each block into row 0 of its slot
-        float* npart = reinterpret_cast<float*>(smem + abytes + (size_t)nwaves * T * 1024);
+        // add_rmsnorm of the one row (lane l: elements 2l, 2l + 1 of this
+        // wave's live blocks).  The factor 1 / rms needs every wave's sum of
+        // v^2, but it is one number: it is left out here and multiplies the
+        // GEMV's result, so no wave waits for another's copies of x before
+        // its first MFMA, and the double arithmetic of 1 / rms is off the way
+        // to it (a captured decode layer with the 6144 x 4096 and the SwiGLU
+        // 24576 x 4096 form, 40.6 -> 39.1 us).  In its place each wave scales
+        // its h by a power of two of its own, from the largest exponent of v
+        // plus that of w, so that |h| < 2^12 and h's rounding to fp16 is
+        // relative to v w as it was; the waves' powers meet in the reduction.
+        // A weight of zero counts as fp16's smallest, 2^-24 (biased 103), so
+        // that the scaled v stays below 2^35 there.
         float ss = 0.0f;
-        float2 v[NB];
+        int ex = 0;  // largest sum of the two biased exponents
+        float2 v[NB], wf[NB];
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
             const unsigned char* sl = aslot + (size_t)i * 1024;
             const float2 xv = *reinterpret_cast<const float2*>(sl + 8 * lane);
             const uint32_t dv = *reinterpret_cast<const uint32_t*>(sl + 512 + 4 * lane);
+            const uint32_t wv2 = *reinterpret_cast<const uint32_t*>(sl + 768 + 4 * lane);
             v[i].x = xv.x + (float)bitcast<f16>((uint16_t)(dv & 0xFFFFu));
             v[i].y = xv.y + (float)bitcast<f16>((uint16_t)(dv >> 16));
+            wf[i].x = (float)bitcast<f16>((uint16_t)(wv2 & 0xFFFFu));
+            wf[i].y = (float)bitcast<f16>((uint16_t)(wv2 >> 16));
             if (i < nb) {
                 ss = __builtin_fmaf(v[i].x, v[i].x, ss);
                 ss = __builtin_fmaf(v[i].y, v[i].y, ss);
             }
+            const auto be = [](float f) { return (int)((__float_as_uint(f) >> 23) & 0xFFu); };
+            const auto bw = [&](float f) { return be(f) > 103 ? be(f) : 103; };
+            const int e0 = be(v[i].x) + bw(wf[i].x), e1 = be(v[i].y) + bw(wf[i].y);
+            ex = ex > e0 ? ex : e0;
+            ex = ex > e1 ? ex : e1;
         }
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
-        if (lane == 0) npart[wave] = ss;
-        lds_barrier();
-        // the partials in wave order: four 16-byte reads (the launch gives
-        // npart 64 floats, so all 16 slots are in the allocation), slots of
-        // absent waves masked -- not one dependent LDS read per wave
-        float pw[16];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float4 f = reinterpret_cast<const float4*>(npart)[q];
-            pw[4 * q] = f.x;
-            pw[4 * q + 1] = f.y;
-            pw[4 * q + 2] = f.z;
-            pw[4 * q + 3] = f.w;
+        for (int off = 32; off > 0; off >>= 1) {
+            const int o = __shfl_xor(ex, off, 64);
+            ex = ex > o ? ex : o;
         }
-        float tot = 0.0f;
-#pragma unroll
-        for (int w = 0; w < 16; ++w) tot += w < nwaves ? pw[w] : 0.0f;
-        const float inv = (float)(1.0 / sqrt((double)tot / (double)K + (double)nrm.eps));
-        uint32_t hv[NB];
+        // |v w| < 2^(ex - 254 + 2), so 2^up brings it below 2^12
+        const int up = 12 - (ex - 252);
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
-            const uint32_t wv2 = *reinterpret_cast<const uint32_t*>(aslot + (size_t)i * 1024 + 768 + 4 * lane);
-            float y0 = v[i].x * inv * (float)bitcast<f16>((uint16_t)(wv2 & 0xFFFFu));
-            float y1 = v[i].y * inv * (float)bitcast<f16>((uint16_t)(wv2 >> 16));
-            // rounded to fp32 first, as the reference does (no fused
-            // multiply-and-convert)
-            asm volatile("" : "+v"(y0), "+v"(y1));
-            hv[i] = (uint32_t)bitcast<uint16_t>((f16)y0) | ((uint32_t)bitcast<uint16_t>((f16)y1) << 16);
+            const float y0 = ldexpf(v[i].x, up) * wf[i].x, y1 = ldexpf(v[i].y, up) * wf[i].y;
+            *reinterpret_cast<uint32_t*>(aslot + (size_t)i * 1024 + 4 * lane) =
+                (uint32_t)bitcast<uint16_t>((f16)y0) | ((uint32_t)bitcast<uint16_t>((f16)y1) << 16);
         }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int i = 0; i < NB; ++i) *reinterpret_cast<uint32_t*>(aslot + (size_t)i * 1024 + 4 * lane) = hv[i];
         if (blockIdx.x == 0) {
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
                 const int kb = wave + i * nwaves;
                 if (i < nb) *reinterpret_cast<float2*>(nrm.xnew + kb * 128 + 2 * lane) = v[i];
             }
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+        if (lane == 0) {
+            npart[wave] = ss;
+            nexp[wave] = up;
         }
     }
     if (ALDS) {
@@ -736,6 +753,30 @@ __device__ __forceinline__ void int4_gemv_body(const f16* __restrict__ A, const 
     for (int t = 0; t < T; ++t)
         *reinterpret_cast<f32x4*>(red + (wave * T + t) * 256 + lane * 4) = acc[t];
     __syncthreads();
+    // AM 4: 1 / rms from the waves' sums in wave order, and the smallest of
+    // their powers of two, to which the partials are brought (down, so none
+    // overflows): the sum times `fin` is the result
+    float fin = 1.0f;
+    int emin = 0;
+    if (AM == 4) {
+        // all 16 slots in 16-byte reads, those of absent waves masked -- not
+        // one dependent LDS read per wave
+        float tot = 0.0f;
+        emin = nexp[0];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 p4 = reinterpret_cast<const f32x4*>(npart)[q];
+            const i32x4_t e4 = reinterpret_cast<const i32x4_t*>(nexp)[q];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const bool there = 4 * q + r < nwaves;
+                tot += there ? p4[r] : 0.0f;
+                emin = there && e4[r] < emin ? e4[r] : emin;
+            }
+        }
+        fin = ldexpf(inv_rms(tot, nrm.rk, nrm.eps), -emin);
+    }
+    const auto part = [&](int w, int i) { return AM == 4 ? ldexpf(red[i], emin - nexp[w]) : red[i]; };
     if (SWI) {
         for (int idx = threadIdx.x; idx < 256; idx += blockDim.x) {
             const int l = idx >> 2, e = idx & 3;
@@ -743,8 +784,12 @@ __device__ __forceinline__ void int4_gemv_body(const f16* __restrict__ A, const 
             if (m >= M) continue;
             float g = 0.f, u = 0.f;
             for (int w = 0; w < nwaves; ++w) {
-                g += red[(w * T) * 256 + idx];
-                u += red[(w * T + 1) * 256 + idx];
+                g += part(w, (w * T) * 256 + idx);
+                u += part(w, (w * T + 1) * 256 + idx);
+            }
+            if (AM == 4) {
+                g *= fin;
+                u *= fin;
             }
             const float gf = (float)(f16)g, uf = (float)(f16)u;
             C[(size_t)m * (N >> 1) + strip * 16 + (l & 15)] = (f16)(gf / (1.0f + expf(-gf)) * uf);
@@ -757,7 +802,8 @@ __device__ __forceinline__ void int4_gemv_body(const f16* __restrict__ A, const 
             const int m = 4 * (l >> 4) + e;
             if (m >= M) continue;
             float v = 0.f;
-            for (int w = 0; w < nwaves; ++w) v += red[(w * T + t) * 256 + (idx & 255)];
+            for (int w = 0; w < nwaves; ++w) v += part(w, (w * T + t) * 256 + (idx & 255));
+            if (AM == 4) v *= fin;
             C[(size_t)m * N + (strip * T + t) * 16 + (l & 15)] = (f16)v;
         }
         return;
@@ -1859,7 +1905,7 @@ int fastllm_int4_gemm_add_rmsnorm(const float* x, const void* delta, const void*
         return 1;
     if (!fl_current_device_supported()) return 2;
     const NormArgs nrm{x, static_cast<const uint16_t*>(delta), static_cast<const uint16_t*>(norm_w), xnew,
-                       eps};
+                       eps, 1.0 / size_k};
     const uint16_t* S = static_cast<const uint16_t*>(b_scales);
     f16* C = static_cast<f16*>(c);
     const hipError_t e =

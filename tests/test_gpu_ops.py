@@ -113,6 +113,60 @@ def test_gemm_add_rmsnorm(torch_gpu, N, K, gs, swiglu):
         assert Q.max_abs_rel(got, two.float().cpu().numpy()) < 5e-3
 
 
+@pytest.mark.parametrize("kind", ["plain", "outliers", "blocks far apart", "tiny", "zero", "large weights",
+                                  "zero weights", "huge"])
+@pytest.mark.parametrize("N,K,swiglu", [(192, 384, False), (6144, 4096, False), (256, 2048, True)])
+def test_gemm_add_rmsnorm_ranges(torch_gpu, kind, N, K, swiglu):
+    """Rows whose blocks differ by many orders of magnitude: every wave scales
+    its h by a power of two of its own.  Against float64, with h's and the
+    result's rounding to fp16 and K fp32 additions as the bound; a row whose
+    sum of squares overflows gives zeros."""
+    from fastllm_py.kernels import marlin
+
+    torch = torch_gpu
+    rng = np.random.default_rng(700 + N + K)
+    W = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    from fastllm_py.moe import quantize_marlin_matrix_device
+    pay = quantize_marlin_matrix_device(torch.from_numpy(W).cuda(), 128)
+    q, s_, z = Q.quantize_int4_marlin(W, 128)
+    w_hat = torch.from_numpy(Q.marlin_dequant(q, *Q.marlin_scales_zeros(s_, z), 128)).cuda().double()
+    x = rng.standard_normal((1, K)).astype(np.float32)
+    d = (rng.standard_normal((1, K)) * 0.5).astype(np.float16)
+    ln = (1.0 + 0.1 * rng.standard_normal(K)).astype(np.float16)
+    if kind == "outliers":
+        x[0, ::97] *= 3e4
+    elif kind == "blocks far apart":
+        x *= np.repeat(10.0 ** rng.integers(-12, 7, K // 128), 128).astype(np.float32)
+        d[:] = 0
+    elif kind in ("tiny", "huge"):
+        x *= np.float32(1e-20 if kind == "tiny" else 1e25)
+        d[:] = 0
+    elif kind == "zero":
+        x[:], d[:] = 0, 0
+    elif kind == "large weights":
+        ln[::5] = 100
+    elif kind == "zero weights":  # all of some waves' blocks
+        ln[K // 3:] = 0
+    xd, dd, lnd = (torch.from_numpy(a).cuda() for a in (x, d, ln))
+    xnew, c = marlin.gemm_add_rmsnorm(xd, dd, lnd, 1e-6, pay["qweight"], pay["scales"], pay["zeros"], N, K,
+                                      swiglu=swiglu)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(xnew.cpu().numpy(), x + d.astype(np.float32))
+    if kind == "huge":
+        assert torch.count_nonzero(c).item() == 0
+        return
+    v = xd.double() + dd.double()
+    h = v / torch.sqrt((v * v).mean() + 1e-6) * lnd.double()
+    ref, mag = h @ w_hat.T, h.abs() @ w_hat.abs().T
+    err = 2.0 ** -11 * ref.abs() + (2.0 ** -11 + K * 2.0 ** -24) * mag + 2.0 ** -24
+    if swiglu:
+        g, u = ref.chunk(2, -1)
+        eg, eu = err.chunk(2, -1)
+        ref = g / (1 + torch.exp(-g)) * u  # |silu'| <= 1.1, |silu(g)| <= |g|
+        err = 1.1 * eg * (u.abs() + eu) + g.abs() * eu + 2.0 ** -10 * ref.abs() + 2.0 ** -24
+    assert ((c.double() - ref).abs() <= err).all()
+
+
 def test_gemm_add_rmsnorm_rejects(torch_gpu):
     from fastllm_py import _native as nat
 
