@@ -2806,27 +2806,23 @@ __global__ __launch_bounds__(256) void moe_combine_k(MoeArgs a) {
 // from inline asm, see common.cuh), kMgAhead blocks ahead, into a ring of
 // kMgAhead + 1 stages; one vmcnt wait and one barrier per 128-k block hand
 // a stage to all waves.  One block ahead in two stages (two workgroups per
-// CU): config 5 148.8-154.2 us per layer, against 190.9 us two blocks ahead
-// in three stages (one workgroup per CU).  A stage holds
-//   * A (16 KB): 64 rows x 128 k fp16.  FP8 / MXFP4: row-major (256 B per
-//     row) with the 16-byte k chunks of row r XOR-swizzled by r % 16, so
-//     each copy moves 4 whole rows and the 16 lanes of an MFMA operand read
-//     hit 16 different bank groups -- lane (c, q) of MFMA step j of m-tile
-//     mt reads row 16 mt + c, chunk a_koff(q, j) / 8 at position chunk ^ c.
-//     INT4: fragment-major -- lane (c, q) of MFMA step j reads row c, k
-//     32 q + 8 j .. + 7 at 16 (64 (4 mt + j) + c + 16 q);
-//   * per wave (2.5 KB): its two 1 KB tile blocks and the tiles' 16 x
-//     (128 / gs) scale|zero words.
-// B is dequantized in registers to s * (q - z) in fp16 (lane (c, q)'s 32 k
-// lie in one group for every group size >= 32) and 32 MFMAs per wave and
+// CU) beats two ahead in three (one per CU): 150 against 191 us for 512 tokens
+// over 128 experts.  moe_gemm_k is the MXFP4 form; INT4 (moe_gemm_rk) and FP8
+// (moe_gemm_wide) experts keep their weights in registers.  A stage holds
+//   * A (16 KB): 64 rows x 128 k fp16, row-major (256 B per row) with the
+//     16-byte k chunks of row r XOR-swizzled by r % 16, so each copy moves 4
+//     whole rows and the 16 lanes of an MFMA operand read hit 16 different
+//     bank groups -- lane (c, q) of MFMA step j of m-tile mt reads row
+//     16 mt + c, chunk a_koff(q, j) / 8 at position chunk ^ c;
+//   * per wave (2.5 KB): its two 1 KB tile blocks and their E8M0 words.
+// B is the code times its MX block's scale in fp16 and 32 MFMAs per wave and
 // block accumulate in fp32; m-tiles past the chunk's rows skip their MFMAs.
 constexpr int kMgAhead = 1, kMgStages = kMgAhead + 1;
 constexpr int kMgWaves = 8;                     // waves per workgroup
-// per wave and stage: two tile blocks (1 KB, FP8 2 KB) + two 256-byte scale rows
-constexpr int mg_wave_stage(int fmt) { return 2 * (fmt == kFmtFp8 ? 2048 : 1024) + 2 * 256; }
+constexpr int kMgWaveStage = 2 * 1024 + 2 * 256;  // per wave: two tile blocks, two 256-byte scale rows
 constexpr int kMgABytes = 64 * 128 * 2;            // A tile of one stage
-constexpr int mg_stage(int fmt) { return kMgABytes + kMgWaves * mg_wave_stage(fmt); }
-constexpr size_t mg_lds(int fmt) { return (size_t)kMgStages * mg_stage(fmt); }
+constexpr int kMgStage = kMgABytes + kMgWaves * kMgWaveStage;
+constexpr size_t kMgLds = (size_t)kMgStages * kMgStage;
 
 // xh[t, :] = fp16(x[t, :]) for the grouped kernels' A copies
 __global__ void x_to_f16_k(const float* __restrict__ x, uint16_t* __restrict__ xh, int n8) {
@@ -2883,20 +2879,12 @@ FL_DEV MgUnit mg_unit(const MoeArgs& a) {
     return MgUnit{y / a.nch_r, strip, y % a.nch_r * 64, a.nch_r * 64, 0, -1};
 }
 
-template <int PHASE, bool G128, int FMT = kFmtInt4>
+template <int PHASE>
 __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int D = kMgAhead, NS = kMgStages;
     constexpr int NW = kMgWaves, FPW = 16 / NW;  // waves, A fragments copied per wave
-    constexpr int BPT = FMT == kFmtFp8 ? 2 : 1;  // 1 KB copies per tile block
-    constexpr int TB = 1024 * BPT;               // tile block bytes
-    constexpr int WST = mg_wave_stage(FMT), STG = mg_stage(FMT);
-    constexpr int LPB = FPW + 2 * BPT + 2;  // per block and wave: A fragments, B copies, 2 scale rows
-    // FP8 / MXFP4 stage A row-major in whole rows (config 5: FP8 204 -> 198,
-    // MXFP4 150 -> 147 us per layer); INT4 keeps the MFMA fragment order,
-    // whose reads need no per-step lane addressing (its dequantization keeps
-    // the VALU busy: 146 against 160 us with whole rows)
-    constexpr bool ROWA = FMT != kFmtInt4;
+    constexpr int LPB = FPW + 2 + 2;  // per block and wave: A fragments, B copies, 2 scale rows
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, kq = lane >> 4;
@@ -2930,8 +2918,6 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
     if (un.mc >= M || strip * ncols >= Nrows) return;
     const int nkb_all = K >> 7, nkb = un.kbn < 0 ? nkb_all : un.kbn;  // the weight's blocks, this unit's
     if (nkb <= 0) return;
-    const int G = K / a.gs;
-    const int spb = 128 / a.gs;  // groups per 128-k block
 
     // this wave's two weight tiles
     i32x4_t rq[2], rz[2];
@@ -2949,13 +2935,8 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
             tq = ex->dq;
             tsz = ex->dsz;
         }
-        rq[t] = raw_rsrc(tq + (tile * nkb_all + un.kb0) * TB, nkb * TB);
-        if (FMT == kFmtFp8)  // one fp32 scale per (128-row band, block)
-            rz[t] = raw_rsrc(tsz + (tile >> 3) * nkb_all + un.kb0, nkb * 4);
-        else if (FMT == kFmtMx4)  // 16 E8M0 words per block
-            rz[t] = raw_rsrc(tsz + (tile * nkb_all + un.kb0) * 16, nkb * 64);
-        else
-            rz[t] = raw_rsrc(tsz + (tile * G + un.kb0 * spb) * 16, nkb * spb * 64);
+        rq[t] = raw_rsrc(tq + (tile * nkb_all + un.kb0) * 1024, nkb * 1024);
+        rz[t] = raw_rsrc(tsz + (tile * nkb_all + un.kb0) * 16, nkb * 64);  // 16 E8M0 words per block
     }
     // A rows: PHASE 0 token rows of xh, PHASE 1 the slot's inter_buf rows
     const uint16_t* abase = PHASE == 0 ? a.xh : a.inter_buf;
@@ -2963,21 +2944,14 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
     const int arows = PHASE == 0 ? a.T : a.max_entries + a.T;
     const i32x4_t rA = raw_rsrc(abase, (uint32_t)arows * astride * 2);
     const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
-    // scale-row copy: INT4 16 words per group, MXFP4 16 words, FP8 the one
-    // block scale (every lane copies it)
-    const uint32_t zlane = FMT == kFmtFp8 ? 0u
-                         : FMT == kFmtMx4 ? 4u * (lane < 16 ? lane : 15)
-                                          : 4u * (lane < 16 * spb ? lane : 16 * spb - 1);
-    const int zstep = FMT == kFmtFp8 ? 4 : (FMT == kFmtMx4 ? 64 : spb * 64);  // scale bytes per block
-    const int g_local = kq * 32 / a.gs;  // this lane's group within a block
+    const uint32_t zlane = 4u * (lane < 16 ? lane : 15);  // scale-row copy: 16 words
 
     for (int mc = un.mc; mc < M; mc += un.mstep) {
         const int mt_live = (M - mc + 15) >> 4;  // m-tiles holding rows of this chunk
-        // A copies f = FPW wave + i of this wave.  FP8 / MXFP4 (ROWA): chunk
-        // rows 4 f .. 4 f + 3 (m-tile f / 4), each the row's whole 256 bytes
-        // of the block (two full cache lines); lane l takes row 4 f + l / 16
-        // and its 16-byte k chunk (l % 16) ^ (row % 16).  INT4: fragment f =
-        // 4 m-tile + j in MFMA order (16 rows x four 16-byte pieces).
+        // A copies f = FPW wave + i of this wave: chunk rows 4 f .. 4 f + 3
+        // (m-tile f / 4), each the row's whole 256 bytes of the block (two
+        // full cache lines); lane l takes row 4 f + l / 16 and its 16-byte k
+        // chunk (l % 16) ^ (row % 16).
         // lane l holds row mc + l's token and combine weight (rows past M
         // repeat row M - 1), read once per chunk and handed out by shuffles
         const int ml = mc + lane < M ? mc + lane : M - 1;
@@ -2987,31 +2961,27 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
 #pragma unroll
         for (int i = 0; i < FPW; ++i) {
             const int f = wave * FPW + i;
-            const int r = ROWA ? 4 * f + (lane >> 4) : 16 * (f >> 2) + col;
+            const int r = 4 * f + (lane >> 4);
             int m = mc + r;
             m = m < M ? m : M - 1;
             const int row = PHASE == 0 ? __shfl(ltok, m - mc, 64) : row0 + m;
-            ao[i] = 2u * ((uint32_t)row * astride + 128u * un.kb0 +
-                          (ROWA ? 8 * ((lane & 15) ^ (r & 15)) : a_koff<FMT>(kq, f & 3)));
+            ao[i] = 2u * ((uint32_t)row * astride + 128u * un.kb0 + 8 * ((lane & 15) ^ (r & 15)));
         }
         // blocks past the end keep the copy count with lane offsets past
         // every buffer's range: they read zeros without touching memory
         auto issue = [&](int kb, int stg) {
             const uint32_t oob = kb < nkb ? 0u : 0x80000000u;
             kb = kb < nkb ? kb : nkb - 1;
-            const uint32_t st = lds0 + (uint32_t)stg * STG;
+            const uint32_t st = lds0 + (uint32_t)stg * kMgStage;
 #pragma unroll
             for (int i = 0; i < FPW; ++i)
                 if (kMgAhead > 1 || wave * FPW + i < 4 * mt_live)  // dead m-tiles: no copy
                     lds_copy(rA, st + (wave * FPW + i) * 1024, ao[i] | oob, kb * 256);
-            const uint32_t wst = st + kMgABytes + wave * WST;
+            const uint32_t wst = st + kMgABytes + wave * kMgWaveStage;
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+            for (int t = 0; t < 2; ++t) lds_copy(rq[t], wst + t * 1024, (lane * 16) | oob, kb * 1024);
 #pragma unroll
-                for (int h = 0; h < BPT; ++h)  // FP8: the block's two 1 KB halves
-                    lds_copy(rq[t], wst + t * TB + h * 1024, (h * 1024 + lane * 16) | oob, kb * TB);
-#pragma unroll
-            for (int t = 0; t < 2; ++t) lds_copy<4>(rz[t], wst + 2 * TB + t * 256, zlane | oob, kb * zstep);
+            for (int t = 0; t < 2; ++t) lds_copy<4>(rz[t], wst + 2048 + t * 256, zlane | oob, kb * 64);
         };
 
         f32x4 acc[4][2];
@@ -3026,109 +2996,31 @@ __global__ __launch_bounds__(64 * kMgWaves) void moe_gemm_k(MoeArgs a) {
             wait_vmcnt<(D - 1) * LPB>();
             asm volatile("s_barrier" ::: "memory");
             issue(kb + D, (kb + D) % NS);
-            const unsigned char* st = smem + (size_t)(kb % NS) * STG;
-            const unsigned char* wst = st + kMgABytes + wave * WST;
-            if constexpr (FMT != kFmtInt4) {
-                // FP8 / MXFP4: codes to fp16 once per (tile, step) for the
-                // four m-tiles; FP8 scales the block's partial once, MXFP4
-                // every step (one MX block per step)
-                WBlk<FMT> bl[2];
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    bl[t].w = *reinterpret_cast<const u32x4*>(wst + t * TB + lane * 16);
-                    if (FMT == kFmtFp8) bl[t].w2 = *reinterpret_cast<const u32x4*>(wst + t * TB + 1024 + lane * 16);
-                    bl[t].sz = *reinterpret_cast<const uint32_t*>(wst + 2 * TB + t * 256 +
-                                                                  (FMT == kFmtMx4 ? 4 * col : 0));
-                }
-                const unsigned char* ab = st + col * 256;  // ROWA (FP8 / MXFP4)
-                f32x4 part[4][2];
-#pragma unroll
-                for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-                    for (int t = 0; t < 2; ++t) part[mt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    f16x8 av[4];
-#pragma unroll
-                    for (int mt = 0; mt < 4; ++mt)
-                        av[mt] = *reinterpret_cast<const f16x8*>(ab + mt * 4096 + 16 * ((a_koff<FMT>(kq, j) >> 3) ^ col));
-#pragma unroll
-                    for (int t = 0; t < 2; ++t) {
-                        if (FMT == kFmtMx4) {
-                            const f16x8 b = mx_operand_scaled(bl[t].w[j], mx_step_scale(bl[t].sz, j));
-#pragma unroll
-                            for (int mt = 0; mt < 4; ++mt)
-                                if (mt < mt_live) acc[mt][t] = mfma_f16(av[mt], b, acc[mt][t]);
-                        } else {
-                            const f16x8 b = wblk_operand(bl[t], j);
-#pragma unroll
-                            for (int mt = 0; mt < 4; ++mt)
-                                if (mt < mt_live) part[mt][t] = mfma_f16(av[mt], b, part[mt][t]);
-                        }
-                    }
-                }
-                if (FMT == kFmtFp8) {
-#pragma unroll
-                    for (int t = 0; t < 2; ++t) {
-                        const float sv = __uint_as_float(bl[t].sz);
-#pragma unroll
-                        for (int mt = 0; mt < 4; ++mt)
-                            if (mt < mt_live)
-#pragma unroll
-                                for (int i = 0; i < 4; ++i) acc[mt][t][i] = __builtin_fmaf(sv, part[mt][t][i], acc[mt][t][i]);
-                    }
-                }
-                continue;
-            }
-            u32x4 wv[2];
-            uint32_t zlo[2], zhi[2];
-            uint16_t sc[2];
+            const unsigned char* st = smem + (size_t)(kb % NS) * kMgStage;
+            const unsigned char* wst = st + kMgABytes + wave * kMgWaveStage;
+            // codes to fp16, scaled, once per (tile, step = one MX block) for
+            // the four m-tiles
+            u32x4 bw[2];
+            uint32_t bs[2];
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                wv[t] = *reinterpret_cast<const u32x4*>(wst + t * 1024 + lane * 16);
-                const uint32_t szw =
-                    *reinterpret_cast<const uint32_t*>(wst + 2048 + t * 256 + 4 * (g_local * 16 + col));
-                tile_zero_bits(sz_zero(szw), zlo[t], zhi[t]);
-                sc[t] = sz_scale(szw);
+                bw[t] = *reinterpret_cast<const u32x4*>(wst + t * 1024 + lane * 16);
+                bs[t] = *reinterpret_cast<const uint32_t*>(wst + 2048 + t * 256 + 4 * col);
             }
-            const unsigned char* ab = st + lane * 16;  // INT4: fragment order
-            // group 128: q - z products accumulate in a per-block fp32 partial
-            // that takes the column scale once; smaller groups scale B in fp16
-            f32x4 part[4][2];
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-                for (int t = 0; t < 2; ++t) part[mt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const unsigned char* ab = st + col * 256;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 f16x8 av[4];
 #pragma unroll
                 for (int mt = 0; mt < 4; ++mt)
-                    av[mt] = *reinterpret_cast<const f16x8*>(ab + (mt * 4 + j) * 1024);
+                    av[mt] = *reinterpret_cast<const f16x8*>(ab + mt * 4096 +
+                                                             16 * ((a_koff<kFmtMx4>(kq, j) >> 3) ^ col));
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    f16x8 b = dequant_word_fast(wv[t][j], zlo[t], zhi[t], 0x64006400u, 0x54005400u);
-                    if (!G128) b = bitcast<f16x8>(scale_f16x8(bitcast<u32x4>(b), sc[t]));
+                    const f16x8 b = mx_operand_scaled(bw[t][j], mx_step_scale(bs[t], j));
 #pragma unroll
                     for (int mt = 0; mt < 4; ++mt)
-                        if (mt < mt_live) {
-                            if (G128)
-                                part[mt][t] = mfma_f16(av[mt], b, part[mt][t]);
-                            else
-                                acc[mt][t] = mfma_f16(av[mt], b, acc[mt][t]);
-                        }
-                }
-            }
-            if (G128) {
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const float sv = (float)bitcast<f16>(sc[t]);
-#pragma unroll
-                    for (int mt = 0; mt < 4; ++mt)
-                        if (mt < mt_live)
-#pragma unroll
-                            for (int i = 0; i < 4; ++i)
-                                acc[mt][t][i] = __builtin_fmaf(sv, part[mt][t][i], acc[mt][t][i]);
+                        if (mt < mt_live) acc[mt][t] = mfma_f16(av[mt], b, acc[mt][t]);
                 }
             }
         }
@@ -3918,8 +3810,8 @@ void launch_grouped_pair(const MoeArgs& gu, const MoeArgs& dn, hipStream_t st) {
         hipLaunchKernelGGL((moe_gemm_rk<1, G128>), grid(dn), dim3(64 * kMgWaves), (size_t)(kMrD + 1) * kMgABytes, st,
                            dn);
     } else {
-        hipLaunchKernelGGL((moe_gemm_k<0, G128, FMT>), grid(gu), dim3(64 * kMgWaves), mg_lds(FMT), st, gu);
-        hipLaunchKernelGGL((moe_gemm_k<1, G128, FMT>), grid(dn), dim3(64 * kMgWaves), mg_lds(FMT), st, dn);
+        hipLaunchKernelGGL((moe_gemm_k<0>), grid(gu), dim3(64 * kMgWaves), kMgLds, st, gu);
+        hipLaunchKernelGGL((moe_gemm_k<1>), grid(dn), dim3(64 * kMgWaves), kMgLds, st, dn);
     }
 }
 
