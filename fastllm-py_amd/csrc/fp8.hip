@@ -725,15 +725,19 @@ Fp8Cfg fp8_cfg(int M, int N, int K) {
 
 constexpr size_t kFp8LdsCap = 96 * 1024;
 
-// Split-K FP8 GEMM (M > kF8MinM, 128 x 128 block format, few output tiles and
-// long K; other shapes above 16 rows take fp8_gemm_b128, fp8_gemm.hip).
-//   * Workgroup tile 64 (m) x 128 (n), eight waves side by side along n, a
-//     64 x 16 wave tile (four m-tiles x one n-tile of 16 x 16 fp32).
+// Prefill-shaped FP8 GEMM (128 x 128 block format, kF8MinM < M <
+// kF8WideRows; other shapes above 16 rows take fp8_gemm_b128, fp8_gemm.hip).
+//   * Workgroup tile BM (m) x 128 (n), eight waves side by side along n, a
+//     BM x 16 wave tile (BM / 16 m-tiles x one n-tile of 16 x 16 fp32).
+//     BM = 64, or 32 where the 64-row grid has at most 128 tiles and no K
+//     split (2048 x 2048, M = 512: 13.6 -> 10.0 us; the copies bound the
+//     kernel per CU, and twice the workgroups reach every CU for 1.5x the
+//     lines copied in all).
 //   * Every main-loop load goes global -> LDS (lds_copy: buffer_load ...
-//     lds from inline asm) D 128-k blocks ahead into D + 1 stages of 32 KB,
-//     one vmcnt wait and one barrier per block.  With the builtin copies the
-//     compiler drained them all before each block's LDS reads, so no ring
-//     held more than one block.
+//     lds from inline asm) D 128-k blocks ahead into D + 1 stages of 32 KB
+//     (D = 1: two workgroups per CU; D = 3: one), one vmcnt wait and one
+//     barrier per block.  With the builtin copies the compiler drained them
+//     all before each block's LDS reads, so no ring held more than one block.
 //   * A stage holds the 64 x 128 activation tile row-major (256 B per row,
 //     the 16-byte k chunks of row r XOR-swizzled by r % 16) and the strip's
 //     128 weight rows x 128 codes row-major (128 B per row, the 16-code
@@ -743,7 +747,7 @@ constexpr size_t kFp8LdsCap = 96 * 1024;
 //     one without the copies half as long), and a copy that reads 16 rows x
 //     64 B (the fragment-major order this replaced) costs a CU as much as
 //     one of 8 full lines: M = 512, 2048 x 2048 / 10944 x 2048 / 2048 x
-//     10944 19.7 / 56.5 / 53.7 -> 13.6 / 35.6 / 43.6 us.
+//     10944 19.7 / 56.5 / 53.7 -> 13.6 / 35.6 / 43.6 us (ring depths below).
 //   * Codes become fp16/bf16 exactly (v_cvt_scalef32_pk_*_fp8, scale 1); each
 //     block's MFMAs accumulate into a fresh partial that the fp32 block scale
 //     then adds into the accumulator, as the GEMV does.
@@ -755,12 +759,26 @@ constexpr int kF8BM = 64, kF8BN = 128, kF8MinM = 64;
 // measured slower at M = 512: 26.7 / 65.0 / 132.4 us, with half the waves
 // per SIMD to hide the LDS and conversion latencies.
 constexpr int kF8NTW = 1, kF8Waves = 8 / kF8NTW;
-// Blocks in flight ahead of the one computed: 2048 x 10944 in two K splits,
-// M = 512, one / two / three ahead 52.1 / 43.6 / 44.2 us.
-constexpr int kF8Ahead = 3;
-constexpr size_t kF8GemmLds = (size_t)(kF8Ahead + 1) * (kF8BM * 256 + 16384);
+// From this many rows and this many 64 x 128 tiles, fp8_gemm_b128's 32x32 MFMA
+// tiles are the faster ones also with the weights in HBM, not in a cache, as
+// when each layer's are read once.  They hold one block in flight where this
+// kernel's rings hold up to three: below, they are up to 26 % slower there
+// (bf16, weights from HBM, this kernel / those, us: M = 128 2048 x 2048 9.8 /
+// 11.8, 10944 x 2048 14.8 / 16.6; M = 1000 61.2 / 63.9; M = 1536 2048 x 10944
+// 95 / 109, 10944 x 2048 93 / 101; M = 1700 2048 x 10944 (432 tiles) 102 / 110,
+// 10944 x 2048 109 / 104, 4096 x 4096 78 / 62; M = 2000 114 / 113, 121 / 107, 86
+// / 67; M = 4096 228 / 172, 240 / 205, 172 / 133).
+constexpr int kF8WideRows = 1700, kF8WideTiles = 512;
+// Blocks in flight ahead of the one computed (the ring holds D + 1 stages
+// of 32 KB).  Grids of more than 256 workgroups take one block ahead, so
+// two workgroups share a CU; smaller grids (at most one per CU) three.  With
+// whole-line copies, M = 512: 10944 x 2048 (688 workgroups) 35.6 us one
+// ahead, 41.3 two, 39.7 three; 2048 x 2048 (128) 15.7 / 14.7 / 13.6;
+// 2048 x 10944 (two K splits, 256) 52.1 / 43.6 / 44.2.
+// stage = BM x 128 activations (bf16) + 128 x 128 codes
+constexpr size_t fp8_gemm_lds(int ahead, int bm) { return (size_t)(ahead + 1) * (bm * 256 + 16384); }
 
-// Split y of gridDim.y (2 to 4, grids of fewer than 256 tiles) takes 128-k
+// Split-K (gridDim.y > 1, grids of fewer than 256 tiles): split y takes 128-k
 // blocks [y kb_per, (y + 1) kb_per); each split stores its fp32 64 x 128
 // accumulator tile (thread order) with device-coherent stores, waits for
 // them, and bumps the tile's counter; the split that finds gridDim.y - 1
@@ -768,7 +786,7 @@ constexpr size_t kF8GemmLds = (size_t)(kF8Ahead + 1) * (kF8BM * 256 + 16384);
 // resets the counter.  Nothing waits on another workgroup.
 constexpr int kF8TileF = kF8BM * kF8BN;  // fp32 partials per tile and split
 
-template <bool BF16, int D>
+template <bool BF16, int D, int BM = 64>
 __global__ __launch_bounds__(512) void fp8_gemm_mfma(const uint16_t* __restrict__ A,
                                                      const uint8_t* __restrict__ W,
                                                      const float* __restrict__ Sc,
@@ -776,7 +794,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_mfma(const uint16_t* __restrict_
                                                      uint16_t* __restrict__ C, int M, int N, int K,
                                                      int nks, int kb_per, float* __restrict__ part,
                                                      int* __restrict__ cnt) {
-    constexpr int BM = kF8BM;
+    static_assert(BM == 32 || BM == 64, "tile height");
     constexpr int NS = D + 1, NTW = kF8NTW;
     constexpr int AF = BM / 32;          // A copies (4 rows each) per block and wave
     constexpr int MT = BM / 16;          // m-tiles each wave computes
@@ -907,7 +925,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_mfma(const uint16_t* __restrict_
     }
     wait_vmcnt<0>();  // no LDS copy may still be in flight when the workgroup ends
 
-    {
+    if (gridDim.y > 1) {
         static_assert(NTW == 1, "split-K partials assume one n-tile per wave");
         __shared__ int last;
         const int nsplit = (int)gridDim.y;
@@ -1049,29 +1067,38 @@ hipError_t fp8_gemm(const uint16_t* A, const uint8_t* W, const float* Sc, const 
     // M <= 8 there: the halved 8-row kernel (K <= 128 x 2 x 64)
     if (M <= 8 && K >= 512 && K <= 16384 && N < 8192 && N % 8 == 0)
         return fp8_q2<INLINE, BF16>(A, W, Sc, bias, C, M, N, K, rs, nks, st);
-    if (!INLINE && M > 16 && K % 64 == 0 && (size_t)N * K < (1ull << 31) && fp8_gemm_rows(K) > 0) {
-        // few output tiles and long K: the split-K GEMM, where a workspace is
-        // there and its modelled time (5 us for the hand-off, 1 us a block) is
-        // the lower one (2048 x 10944, bf16, M = 128 / 256 / 384: 24 / 26 / 38
-        // us against 37 / 38 / 38)
-        const int s = M > kF8MinM && (size_t)M * K * 2 < (1ull << 31) ? fp8_gemm_splits(M, N, K) : 1;
-        const int nkb = (K + 127) / 128, kb_per = (nkb + s - 1) / s;
-        if (s > 1 && ws && fl_aligned(ws, 256) && ws_bytes >= fp8_gemm_ws_bytes(M, N, K) &&
-            5.0f + kb_per < fp8_gemm_us(M, N, K)) {
-            const int tiles = ((N + kF8BN - 1) / kF8BN) * ((M + kF8BM - 1) / kF8BM);
-            hipLaunchKernelGGL((fp8_gemm_mfma<BF16, kF8Ahead>), dim3(tiles, s), dim3(64 * kF8Waves), kF8GemmLds, st,
-                               A, W, Sc, bias, C, M, N, K, nks, kb_per,
-                               reinterpret_cast<float*>(static_cast<char*>(ws) + kF8CntBytes),
-                               static_cast<int*>(ws));
+    if (!INLINE && M > 16 && K % 64 == 0 && (size_t)N * K < (1ull << 31)) {
+        const int tiles = ((N + kF8BN - 1) / kF8BN) * ((M + kF8BM - 1) / kF8BM);
+        if (M > kF8MinM && (M < kF8WideRows || tiles < kF8WideTiles) && (size_t)M * K * 2 < (1ull << 31)) {
+            const int nkb = (K + 127) / 128;
+            int s = fp8_gemm_splits(M, N, K);
+            if (s > 1 && (!ws || !fl_aligned(ws, 256) || ws_bytes < fp8_gemm_ws_bytes(M, N, K))) s = 1;
+            const int kb_per = (nkb + s - 1) / s;
+            int* cnt = s > 1 ? static_cast<int*>(ws) : nullptr;
+            float* part = s > 1 ? reinterpret_cast<float*>(static_cast<char*>(ws) + kF8CntBytes) : nullptr;
+            if (s == 1 && tiles <= 128) {
+                // at most half the chip with 64-row tiles and no K split: 32-row
+                // tiles, twice the workgroups (1.5x the lines copied in all, but
+                // on every CU)
+                const int t32 = ((N + kF8BN - 1) / kF8BN) * ((M + 31) / 32);
+                hipLaunchKernelGGL((fp8_gemm_mfma<BF16, 3, 32>), dim3(t32, 1), dim3(64 * kF8Waves),
+                                   fp8_gemm_lds(3, 32), st, A, W, Sc, bias, C, M, N, K, nks, kb_per, part, cnt);
+            } else if (tiles * s > 256) {
+                hipLaunchKernelGGL((fp8_gemm_mfma<BF16, 1>), dim3(tiles, s), dim3(64 * kF8Waves), fp8_gemm_lds(1, 64),
+                                   st, A, W, Sc, bias, C, M, N, K, nks, kb_per, part, cnt);
+            } else {
+                hipLaunchKernelGGL((fp8_gemm_mfma<BF16, 3>), dim3(tiles, s), dim3(64 * kF8Waves), fp8_gemm_lds(3, 64),
+                                   st, A, W, Sc, bias, C, M, N, K, nks, kb_per, part, cnt);
+            }
             return hipGetLastError();
         }
         const int rows = fp8_gemm_rows(K);
-        for (int m0 = 0; m0 < M; m0 += rows) {
+        for (int m0 = 0; rows > 0 && m0 < M; m0 += rows) {
             const int Mc = M - m0 < rows ? M - m0 : rows;
             const hipError_t e = fp8_gemm_b128(A + (size_t)m0 * K, W, Sc, bias, C + (size_t)m0 * N, Mc, N, K, BF16, st);
             if (e != hipSuccess) return e;
         }
-        return hipSuccess;
+        if (rows > 0) return hipSuccess;
     }
     // decode-shaped kernel, 16 activation rows per launch
     for (int m0 = 0; m0 < M; m0 += 16) {

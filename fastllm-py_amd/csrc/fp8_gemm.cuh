@@ -9,9 +9,6 @@
 // Most rows of one call for this K (0: none; N K must be below 2^31 too).
 FP8_GEMM_HIDDEN int fp8_gemm_rows(int K);
 
-// Modelled time of fp8_gemm_b128 above 64 rows, in us.
-FP8_GEMM_HIDDEN float fp8_gemm_us(int M, int N, int K);
-
 // C[M, N] = A[M, K] @ dequant(W)^T (+ bias[N]); K % 64 == 0, K >= 128, A and W
 // 16-byte aligned.
 FP8_GEMM_HIDDEN hipError_t fp8_gemm_b128(const uint16_t* A, const uint8_t* W, const float* Sc, const uint16_t* bias,

@@ -271,33 +271,19 @@ void launch_small(const Args& a) {
         launch<BF16, 2, 1, 1, 2, 2, 3>(a);
 }
 
-// Above 64 rows, likewise (us; M 65..2000 at seven N x K: the choice is within
-// 1 % of the fastest of the four on average).  Against 64 x 128 tiles of
-// 16x16x32 MFMAs: 2048 x 2048 / 10944 x 2048 / 2048 x 10944 at 2000 rows 24.9
-// / 113 / 108 -> 21.5 / 95 / 100 us, 2048 x 2048 at 500 rows 18 -> 9.4.
-struct Large {
-    float t[4];
-    int best;
-    explicit Large(const Args& a) {
-        const float nkb = (float)((a.K + 127) >> 7);
-        t[0] = 1.7f + nkb * rounds1(tiles_of(a, 64, 64), 0.42f, 0.46f);
-        t[1] = 1.7f + nkb * rounds1(tiles_of(a, 64, 128), 0.55f, 0.7f);
-        t[2] = 1.5f + nkb * rounds1(tiles_of(a, 64, 256), 1.0f, 1.17f);
-        t[3] = 1.5f + nkb * rounds1(tiles_of(a, 128, 256), 1.55f, 1.95f);
-        best = 0;
-        for (int i = 1; i < 4; ++i)
-            if (t[i] < t[best]) best = i;
-    }
-};
-
+// Above 64 rows (the caller sends 1700 and more), likewise.  Against 64 x 128
+// tiles of 16x16x32 MFMAs, 2000 rows, weights from HBM: 2048 x 2048 / 10944 x
+// 2048 / 2048 x 10944 23.8 / 122 / 115 -> 22.7 / 107 / 113 us; 4096 rows 48 /
+// 240 / 228 -> 38 / 205 / 172.
 template <bool BF16>
 void launch_large(const Args& a) {
-    switch (Large(a).best) {
-        case 0: launch<BF16, 2, 1, 1, 2, 2, 2>(a); break;
-        case 1: launch<BF16, 2, 1, 1, 4, 2, 2>(a); break;
-        case 2: launch<BF16, 2, 1, 1, 8, 1, 1>(a); break;
-        default: launch<BF16, 2, 2, 2, 4, 1, 1>(a); break;
-    }
+    const float nkb = (float)((a.K + 127) >> 7);
+    const float t0 = 1.5f + nkb * rounds1(tiles_of(a, 64, 256), 1.0f, 1.17f);
+    const float t1 = 1.5f + nkb * rounds1(tiles_of(a, 128, 256), 1.55f, 1.95f);
+    if (t0 <= t1)
+        launch<BF16, 2, 1, 1, 8, 1, 1>(a);
+    else
+        launch<BF16, 2, 2, 2, 4, 1, 1>(a);
 }
 
 }  // namespace
@@ -307,11 +293,6 @@ int fp8_gemm_rows(int K) {
     // stay below 2^31
     const long rows = ((1l << 31) - 1) / ((long)K * 2) - 128;
     return rows < 128 ? 0 : (int)(rows / 128 * 128);
-}
-
-float fp8_gemm_us(int M, int N, int K) {
-    const Large l(Args{nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K, nullptr});
-    return l.t[l.best];
 }
 
 hipError_t fp8_gemm_b128(const uint16_t* A, const uint8_t* W, const float* Sc, const uint16_t* bias, uint16_t* C,

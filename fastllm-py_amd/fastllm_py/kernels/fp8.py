@@ -122,7 +122,7 @@ def fp8_gemv_block(x, q, scales, out=None, bias=None, stream=None, workspace=Non
     """128x128-block FP8 GEMV: x [M, K] fp16/bf16, q uint8 [N, K], scales fp32
     [ceil(N/128), ceil(K/128)] (quantizer.quantize_fp8_block's format).
     Returns [M, N] in x's dtype.  K % 64 == 0, K >= 128.  Above 64 rows with
-    fewer than 256 output tiles the GEMM may split K; its partials go to
+    fewer than 256 output tiles the GEMM splits K; its partials go to
     ``workspace`` (a zeroed uint8 device tensor of at least
     fastllm_fp8_b128x128_gemm_ws_bytes bytes) or to a per-device workspace
     shared by calls without one (such calls must not overlap)."""

@@ -341,9 +341,8 @@ int fastllm_fp8_b128x128_gemv(const void *A, const uint8_t *Wq,
                               int M, int N, int K, int isBf16, void *stream);
 
 /* fastllm_fp8_b128x128_gemv with a caller workspace for the prefill GEMM's
- * split-K (M > 64 with fewer than 256 64x128 output tiles, where a long K makes
- * it the faster one by its modelled time: 2048 x 10944 up to M = 256): up to 4
- * splits of the 128-k blocks, each storing fp32 partials;
+ * split-K (M > 64 with fewer than 256 64x128 output tiles: the 2048-wide
+ * outputs): up to 4 splits of the 128-k blocks, each storing fp32 partials;
  * the last split of each tile sums them in split order (deterministic) and
  * writes C.  workspace: fastllm_fp8_b128x128_gemm_ws_bytes(M, N, K) bytes
  * (0: no split for this shape), 256-byte aligned, zero-filled once (the

@@ -191,10 +191,10 @@ def test_fp8_block_gemm_prefill(torch_gpu, M, N, K, bf16):
     (17, 40, 128, True), (33, 1000, 320, False), (64, 2048, 1024, True),  # 32 x 32, six k groups
     (20, 10900, 1984, True), (32, 10900, 2048, False),                    # 32 x 64
     (40, 10900, 192, False), (64, 10944, 1088, True),                     # 64 x 64, three k groups
-    (65, 100, 192, True), (129, 1000, 320, False),                        # 64 x 64, two k groups
-    (100, 10900, 192, True), (66, 10944, 1024, False),                    # 64 x 128
-    (1000, 4090, 192, False), (961, 4096, 640, True),                     # 64 x 256
-    (1000, 6000, 192, True), (900, 6144, 640, False),                     # 128 x 256
+    (65, 100, 192, True), (129, 1000, 320, False), (100, 10900, 192, True),  # 16x16x32 MFMAs
+    (1000, 6000, 192, True), (1699, 6144, 640, False),
+    (1700, 5050, 192, False), (2000, 2048, 640, True),                    # 64 x 256
+    (1700, 2500, 192, True), (1801, 4090, 640, False),                    # 128 x 256
 ])
 def test_fp8_block_gemm_tile_shapes(torch_gpu, M, N, K, bf16):
     """Against the float64 product of the same codes and scales.  Bound: the
