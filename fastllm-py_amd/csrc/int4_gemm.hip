@@ -402,7 +402,8 @@ void launch_small(const Args& a) {
 void launch_large(const Args& a) {
     const float t0 = rounds2(tiles_of(a, 128, 256), 1.85f, 3.2f, 3.55f);
     const int w = tiles_of(a, 256, 192), rem = w % 256;
-    const float t1 = (w / 256) * 2.75f + (rem == 0 ? 0.f : rem <= 128 ? 2.0f : rem <= 200 ? 2.35f : 2.75f);
+    const float t1 = (w / 256) * 2.75f +
+                     (rem == 0 ? 0.f : rem <= 128 && w < 256 ? 2.0f : rem <= 200 ? 2.4f : 2.75f);
     const float t2 = rounds2(tiles_of(a, 128, 128), 1.08f, 1.75f, 1.93f);
     const float t3 = 1.05f * fl_ceil_div(tiles_of(a, 128, 128), 256);
     const float t4 = 0.64f * fl_ceil_div(tiles_of(a, 64, 128), 256);
